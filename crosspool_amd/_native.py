@@ -90,6 +90,10 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "xp_gemm_down": (_INT, [_P, _I64, _I64, _P, _I64, _P, _P, _I64, _P, _SIZE, _P]),
     "xp_gemm_workspace_bytes": (_SIZE, [_I64, _I64, _I64, _INT]),
     "xp_projection": (_INT, [_P, _I64, _I64, _P, _I64, _P, _P, _INT, ctypes.POINTER(ActivationDesc), _P]),
+    "xp_projection_workspace_bytes": (_SIZE, [_I64, _I64, _I64, _INT]),
+    "xp_projection_split": (
+        _INT, [_P, _I64, _I64, _P, _I64, _P, _P, _INT, ctypes.POINTER(ActivationDesc), _P, _SIZE, _P],
+    ),
     "xp_activation": (_INT, [_P, _P, _I64, _I64, _INT, _INT, ctypes.POINTER(ActivationDesc), _P]),
     "xp_dense_workspace_bytes": (_SIZE, [_I64, _I64, _I64]),
     "xp_dense_workspace_layout": (_INT, [_I64, _I64, _I64, ctypes.POINTER(_SIZE)]),

@@ -1306,8 +1306,22 @@ int activation_record(const xp_activation_desc *desc, ActivationArgs &out) {
 
 }  // namespace
 
+size_t xp_projection_workspace_bytes(int64_t rows, int64_t n, int64_t k, int dtype) {
+  const size_t element = dtype_bytes(dtype);
+  if (rows <= 0 || n <= 0 || k <= 0 || element == 0) {
+    return 0;
+  }
+  return projection_scratch_bytes(rows, n, k, static_cast<int>(element));
+}
+
 int xp_projection(const void *x, int64_t rows, int64_t k, const void *w, int64_t n, const float *bias, void *out,
                   int dtype, const xp_activation_desc *activation, xp_stream_t stream) {
+  return xp_projection_split(x, rows, k, w, n, bias, out, dtype, activation, nullptr, 0, stream);
+}
+
+int xp_projection_split(const void *x, int64_t rows, int64_t k, const void *w, int64_t n, const float *bias, void *out,
+                        int dtype, const xp_activation_desc *activation, void *workspace, size_t workspace_bytes,
+                        xp_stream_t stream) {
   XP_REQUIRE(rows >= 0 && k > 0 && n > 0, "projection rows must be non-negative and K, N positive");
   const size_t element = dtype_bytes(dtype);
   XP_REQUIRE(element != 0, "payload dtype must be bf16, fp16 or fp32");
@@ -1323,6 +1337,7 @@ int xp_projection(const void *x, int64_t rows, int64_t k, const void *w, int64_t
   XP_REQUIRE(aligned_to(x, element) && aligned_to(w, element) && aligned_to(out, element) &&
                  (bias == nullptr || aligned_to(bias, 4)),
              "projection operands must be aligned to their element size");
+  XP_REQUIRE(workspace == nullptr || aligned16(workspace), "projection workspace must be 16-byte aligned");
   args.x = x;
   args.w = w;
   args.bias = bias;
@@ -1331,7 +1346,12 @@ int xp_projection(const void *x, int64_t rows, int64_t k, const void *w, int64_t
   args.n = n;
   args.k = k;
   args.dtype = dtype;
-  XP_HIP_CHECK(launch(make_projection(args), static_cast<hipStream_t>(stream)));
+  const ProjectionPlan plan =
+      plan_projection(rows, n, k, static_cast<int>(element), workspace != nullptr ? workspace_bytes : 0);
+  args.partials = plan.ranges > 1 ? static_cast<float *>(workspace) : nullptr;
+  const ProjectionLaunch kernels = make_projection(args, plan, rows, dtype);
+  XP_HIP_CHECK(launch(kernels.main, static_cast<hipStream_t>(stream)));
+  XP_HIP_CHECK(launch(kernels.reduce, static_cast<hipStream_t>(stream)));
   return XP_OK;
 }
 

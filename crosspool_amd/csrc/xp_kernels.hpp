@@ -313,7 +313,31 @@ struct ProjectionArgs {
   int64_t k;
   int32_t dtype;
   ActivationArgs act;
+  float *partials;  // fp32 sums [ranges, rows, n] of K ranges instead of the outputs, or null
+  int64_t k_slice;  // columns per K range (set by make_projection)
 };
+
+// Tile (64 or 128 token and weight rows) and K split of a projection at `rows` rows; a split
+// keeps its sums within `scratch_bytes`.
+struct ProjectionPlan {
+  int tile;
+  int64_t ranges;
+  int64_t k_slice;
+};
+ProjectionPlan plan_projection(int64_t rows, int64_t n, int64_t k, int element_bytes, size_t scratch_bytes);
+// The most scratch plan_projection uses at 64, 128, ... and `capacity` rows (less scratch at
+// another row count only splits K less).
+size_t projection_scratch_bytes(int64_t capacity, int64_t n, int64_t k, int element_bytes);
+
+// The projection and, for a K split, the launch that adds the ranges and applies the epilogue.
+struct ProjectionLaunch {
+  KernelLaunch main;
+  KernelLaunch reduce;
+  int64_t ranges = 1;
+};
+// Grids for `capacity` rows.  x_dtype: the tokens' dtype, args.dtype except for 16-bit tokens
+// against fp32 weights.
+ProjectionLaunch make_projection(const ProjectionArgs &args, const ProjectionPlan &plan, int64_t capacity, int x_dtype);
 
 // output [elements] = activation of inputs ([elements] ungated, [rows, 2 width] gated).
 struct ActivationLaunchArgs {
@@ -326,7 +350,6 @@ struct ActivationLaunchArgs {
   ActivationArgs act;
 };
 
-KernelLaunch make_projection(const ProjectionArgs &args);
 KernelLaunch make_activation(const ActivationLaunchArgs &args);
 
 // ---------------------------------------------------------------- GEMMs

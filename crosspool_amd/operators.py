@@ -195,7 +195,7 @@ class GemmPlan:
             scratch = _native.gemm_workspace_bytes_upto(rows, width, hidden, True)
         else:
             kernel = "projection"
-            scratch = 0
+            scratch = _native.library().xp_projection_workspace_bytes(rows, width, hidden, _DTYPE_CODES[dtype])
         regions = ((torch.uint8, (scratch,)),) if scratch else ()
         return cls(
             input_layout=input_layout,
@@ -247,8 +247,9 @@ class Gemm:
         else:
             desc = None if plan.fused_activation is None else plan.fused_activation.descriptor()
             _native.call(
-                "xp_projection", _ptr(inputs), live, hidden, _ptr(projection.values), width, _ptr(projection.bias),
-                _ptr(output), _DTYPE_CODES[inputs.dtype], None if desc is None else ctypes.byref(desc), _stream(),
+                "xp_projection_split", _ptr(inputs), live, hidden, _ptr(projection.values), width,
+                _ptr(projection.bias), _ptr(output), _DTYPE_CODES[inputs.dtype],
+                None if desc is None else ctypes.byref(desc), scratch, scratch_bytes, _stream(),
             )
 
 

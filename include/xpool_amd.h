@@ -155,6 +155,15 @@ int xp_gemm_down(const void *activated, int64_t rows, int64_t intermediate, cons
 int xp_projection(const void *x, int64_t rows, int64_t k, const void *w, int64_t n, const float *bias, void *out,
                   int dtype, const xp_activation_desc *activation, xp_stream_t stream);
 
+/* xp_projection with scratch for the fp32 sums of K ranges, so that a projection of few rows or
+ * columns is spread over the whole device (GemmPlan's split-K workspace, linear.py:111-131).
+ * `workspace` is 16-byte aligned and may be smaller than xp_projection_workspace_bytes (or null):
+ * K is then split less.  The query is for any row count up to `rows`. */
+size_t xp_projection_workspace_bytes(int64_t rows, int64_t n, int64_t k, int dtype);
+int xp_projection_split(const void *x, int64_t rows, int64_t k, const void *w, int64_t n, const float *bias, void *out,
+                        int dtype, const xp_activation_desc *activation, void *workspace, size_t workspace_bytes,
+                        xp_stream_t stream);
+
 /* Standalone activation over projected bf16 / fp16 values: gated, inputs [rows, 2 * width] in
  * the given Gate/Up order (INTERLEAVED: gate 2j, up 2j + 1; CONCATENATED: gate j, up width + j)
  * and output [rows, width], distinct storage; ungated, inputs and output [rows, width], which

@@ -1,0 +1,100 @@
+"""The general projection at the edges of its tiles, slabs and K ranges.
+
+Against fp64: an fp32 sum of K products differs from the exact one by at most
+``(K + ranges) 2^-24 sum |x w|`` whatever its order; the stored value adds one rounding to the
+payload dtype (at most one ulp once the sum may sit on the other side of a rounding boundary).
+"""
+
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+from crosspool_amd import _native
+
+pytestmark = pytest.mark.gpu
+
+CODES = {torch.bfloat16: _native.XP_DTYPE_BF16, torch.float16: _native.XP_DTYPE_F16, torch.float32: _native.XP_DTYPE_F32}
+MANTISSA = {torch.bfloat16: 7, torch.float16: 10, torch.float32: 23}
+
+
+def _pointer(tensor):
+    return None if tensor is None else ctypes.c_void_p(tensor.data_ptr())
+
+
+def _project(x, w, bias, out, workspace, nbytes):
+    _native.call(
+        "xp_projection_split", _pointer(x), x.shape[0], x.shape[1], _pointer(w), w.shape[0], _pointer(bias),
+        _pointer(out), CODES[x.dtype], None, _pointer(workspace) if nbytes else None, nbytes,
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream),
+    )
+    torch.cuda.synchronize()
+
+
+def _assert_within_bound(out, x, w, bias):
+    exact = x.cpu().double() @ w.cpu().double().t()
+    magnitude = x.cpu().double().abs() @ w.cpu().double().abs().t()
+    if bias is not None:
+        exact += bias.cpu().double()
+        magnitude += bias.cpu().double().abs()
+    sums = (x.shape[1] + 17) * 2.0**-24 * magnitude
+    rounding = exact.abs() * 2.0 ** -MANTISSA[out.dtype] if out.dtype is not torch.float32 else 0.0
+    floor = 2.0**-24 if out.dtype is torch.float16 else 0.0  # half an fp16 subnormal step
+    excess = (out.cpu().double() - exact).abs() - sums - rounding - floor
+    assert bool((excess <= 0).all()), f"largest excess over the bound {excess.max():.3e}"
+
+
+def _operands(device, rows, k, n, dtype, offset=0):
+    generator = torch.Generator(device=device).manual_seed(rows * 131 + k * 17 + n)
+    # `offset` leaves every operand aligned to its element only.
+    x = torch.randn(rows * k + offset, device=device, generator=generator).to(dtype)[offset:].view(rows, k)
+    w = torch.randn(n * k + offset, device=device, generator=generator).to(dtype)[offset:].view(n, k)
+    bias = torch.randn(n, device=device, generator=generator)
+    out = torch.full((rows * n + offset + 16,), 7.0, device=device, dtype=dtype)
+    return x, w, bias, out
+
+
+# Rows and columns around the 64- and 128-row tiles, K around a chunk (8 or 4 columns), a slab
+# (64 or 32) and the K ranges.
+@pytest.mark.parametrize("dtype", tuple(CODES))
+@pytest.mark.parametrize(
+    "rows,k,n",
+    ((1, 1, 1), (1, 7, 3), (63, 9, 65), (64, 64, 64), (65, 63, 66), (3, 65, 129), (129, 31, 2), (2, 33, 63),
+     (5, 1025, 67), (257, 2053, 65), (300, 129, 4097), (1030, 40, 4100)),
+)
+def test_projection_edges(device, dtype, rows, k, n):
+    print(f"projection {dtype} {rows}x{n}x{k}", flush=True)
+    x, w, bias, out = _operands(device, rows, k, n, dtype, offset=1)
+    nbytes = _native.library().xp_projection_workspace_bytes(rows, n, k, CODES[dtype])
+    workspace = torch.full((max(nbytes, 16),), 0xff, device=device, dtype=torch.uint8)
+    _project(x, w, bias, out[1:], workspace, nbytes)
+    _assert_within_bound(out[1: 1 + rows * n].view(rows, n), x, w, bias)
+    assert bool((out[:1] == 7).all()) and bool((out[1 + rows * n:] == 7).all()), "stores outside the output"
+
+
+# A workspace below the query splits K less, down to not at all; every split agrees with fp64.
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float32))
+def test_projection_splits_k_by_its_workspace(device, dtype):
+    rows, k, n = 33, 3001, 130
+    x, w, bias, out = _operands(device, rows, k, n, dtype)
+    full = _native.library().xp_projection_workspace_bytes(rows, n, k, CODES[dtype])
+    plane = rows * n * 4
+    assert full >= 4 * plane
+    for nbytes in (0, plane, 2 * plane + 5, 3 * plane, full):
+        print(f"projection workspace {nbytes} of {full}", flush=True)
+        workspace = torch.full((full,), 0xff, device=device, dtype=torch.uint8)
+        _project(x, w, bias, out, workspace, nbytes)
+        _assert_within_bound(out[: rows * n].view(rows, n), x, w, bias)
+        assert bool((workspace[nbytes:] == 0xff).all()), "sums outside the workspace"
+
+
+def test_projection_keeps_infinities_and_nan_in_their_rows(device):
+    rows, k, n = 70, 77, 66
+    x, w, bias, out = _operands(device, rows, k, n, torch.bfloat16)
+    x[3, 5], x[69, 76], w[65, 0] = float("inf"), float("nan"), float("inf")
+    _project(x, w, bias, out, None, 0)
+    got, expected = out[: rows * n].view(rows, n).float().cpu(), x.float().cpu() @ w.float().cpu().t() + bias.cpu()
+    assert torch.equal(torch.isnan(got), torch.isnan(expected))
+    assert torch.equal(torch.isinf(got), torch.isinf(expected)) and torch.equal(got[torch.isinf(got)], expected[torch.isinf(expected)])
