@@ -65,15 +65,6 @@ __device__ __forceinline__ float payload_round(float value) {
   return P::widen(payload_bits<P>(value));
 }
 
-// The same with the payload chosen at run time (PayloadKind), for the FP32-precision
-// Router logits kernel, whose inner loop is LDS arithmetic.
-__device__ __forceinline__ float payload_widen(uint32_t bits16, int32_t payload) {
-  return payload == kPayloadF16 ? F16Payload::widen(bits16) : Bf16Payload::widen(bits16);
-}
-__device__ __forceinline__ uint32_t payload_bits(float value, int32_t payload) {
-  return payload == kPayloadF16 ? payload_bits<F16Payload>(value) : payload_bits<Bf16Payload>(value);
-}
-
 // ------------------------------------------------------------------ router
 // One wavefront per row; lane l holds experts l, l + 64, ... (PER_LANE each: the fewest of
 // 2, 4, 8 or 16 that cover the expert count, so a 128-expert Router selects over two
@@ -128,10 +119,15 @@ __device__ void router_topk_row(const RouterTopkArgs &a, int64_t row, int lane) 
       const int expert = lane + i * kWave;
       float value = kNegativeInfinity;
       if (expert < experts) {
-        // One rounding of the sum to the payload dtype, stored as the logit.
-        const uint32_t bits = payload_bits<P>(sum[i]);
-        a.logits_out[row * experts + expert] = static_cast<uint16_t>(bits);
-        value = P::widen(bits);
+        if (a.logits_f32 != 0) {
+          static_cast<float *>(a.logits_out)[row * experts + expert] = sum[i];
+          value = sum[i];
+        } else {
+          // One rounding of the sum to the payload dtype, stored as the logit.
+          const uint32_t bits = payload_bits<P>(sum[i]);
+          static_cast<uint16_t *>(a.logits_out)[row * experts + expert] = static_cast<uint16_t>(bits);
+          value = P::widen(bits);
+        }
       }
       logit[i] = value;
       maximum = fmaxf(maximum, value);
@@ -239,69 +235,6 @@ __global__ __launch_bounds__(256) void router_topk_kernel(RouterTopkArgs a) {
   const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (row < a.rows) {
     router_topk_row<PER_LANE, P>(a, row, threadIdx.x & (kWave - 1));
-  }
-}
-
-// Router logits for the FP32 and FP32_LOGITS precisions, and for PAYLOAD when the geometry
-// does not suit the MFMA projection (hidden or expert count not a multiple of 8): a
-// workgroup computes a 16-row x 64-expert block; thread t owns row t / 16 and experts
-// 4 (t % 16) .. + 3, each a sequential fp32 sum over the hidden dimension staged through LDS
-// 64 columns at a time, stored as fp32 or rounded once to the payload dtype.
-__global__ __launch_bounds__(256) void router_logits_kernel(RouterLogitsArgs a) {
-  constexpr int ROWS = 16;
-  constexpr int EXPERTS = 64;
-  constexpr int CHUNK = 64;
-  __shared__ float xs[ROWS][CHUNK + 1];
-  __shared__ float ws[EXPERTS][CHUNK + 1];
-  const int tid = threadIdx.x;
-  const int64_t row0 = static_cast<int64_t>(blockIdx.y) * ROWS;
-  const int expert0 = static_cast<int>(blockIdx.x) * EXPERTS;
-  const int my_row = tid / 16;
-  const int my_expert = (tid % 16) * 4;
-  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int64_t k0 = 0; k0 < a.hidden; k0 += CHUNK) {
-    for (int index = tid; index < ROWS * CHUNK; index += 256) {
-      const int r = index / CHUNK;
-      const int c = index % CHUNK;
-      const int64_t row = row0 + r;
-      xs[r][c] = row < a.rows && k0 + c < a.hidden ? payload_widen(a.x[row * a.hidden + k0 + c], a.payload) : 0.0f;
-    }
-    for (int index = tid; index < EXPERTS * CHUNK; index += 256) {
-      const int e = index / CHUNK;
-      const int c = index % CHUNK;
-      const int expert = expert0 + e;
-      float value = 0.0f;
-      if (expert < a.experts && k0 + c < a.hidden) {
-        const int64_t offset = static_cast<int64_t>(expert) * a.hidden + k0 + c;
-        value = a.weights_f32 != 0 ? static_cast<const float *>(a.w)[offset]
-                                   : payload_widen(static_cast<const uint16_t *>(a.w)[offset], a.payload);
-      }
-      ws[e][c] = value;
-    }
-    __syncthreads();
-    const int columns = a.hidden - k0 < CHUNK ? static_cast<int>(a.hidden - k0) : CHUNK;
-    for (int c = 0; c < columns; ++c) {
-      const float x = xs[my_row][c];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        acc[j] = fmaf(x, ws[my_expert + j][c], acc[j]);
-      }
-    }
-    __syncthreads();
-  }
-  const int64_t row = row0 + my_row;
-  if (row < a.rows) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int expert = expert0 + my_expert + j;
-      if (expert < a.experts) {
-        if (a.out_payload != 0) {
-          static_cast<uint16_t *>(a.logits)[row * a.experts + expert] = static_cast<uint16_t>(payload_bits(acc[j], a.payload));
-        } else {
-          static_cast<float *>(a.logits)[row * a.experts + expert] = acc[j];
-        }
-      }
-    }
   }
 }
 
@@ -612,11 +545,6 @@ KernelLaunch make_router_topk(const RouterTopkArgs &args) {
   const void *kernel = args.payload == kPayloadF16 ? router_topk_kernel_for<F16Payload>(per_lane)
                                                    : router_topk_kernel_for<Bf16Payload>(per_lane);
   return launch_of(kernel, dim3(blocks_for(args.rows, 4)), 256, args);
-}
-
-KernelLaunch make_router_logits(const RouterLogitsArgs &args) {
-  return launch_of(reinterpret_cast<const void *>(&router_logits_kernel),
-                   dim3(blocks_for(args.experts, 64), blocks_for(args.rows, 16)), 256, args);
 }
 
 KernelLaunch make_finalize_routing(const FinalizeRoutingArgs &args) {

@@ -506,6 +506,9 @@ ProjectionPlan plan_projection(int64_t rows, int64_t n, int64_t k, int element_b
   const int64_t slab = kSlabBytes / element_bytes;
   const int64_t slabs = (k + slab - 1) / slab;
   const int64_t plane_bytes = rows * n * 4;
+  // Priced at whole 64-row tiles: the choice then changes only with their number, which makes
+  // projection_scratch_bytes exact.
+  const int64_t whole_plane_bytes = (rows + 63) / 64 * 64 * n * 4;
   ProjectionPlan best{64, 1, k};
   double best_us = -1.0;
   for (const ProjectionCost &cost : element_bytes == 4 ? kProjectionCosts32 : kProjectionCosts16) {
@@ -521,7 +524,7 @@ ProjectionPlan plan_projection(int64_t rows, int64_t n, int64_t k, int element_b
       const double rounds = cost.tile == 64 ? std::ceil(per_cu) : per_cu;
       double us = static_cast<double>(per_range) * std::max(cost.latency, rounds * cost.throughput);
       if (ranges > 1) {
-        us += kProjectionReduceUs + 2.0 * static_cast<double>(ranges * plane_bytes) / kProjectionPartialBytesPerUs;
+        us += kProjectionReduceUs + 2.0 * static_cast<double>(ranges * whole_plane_bytes) / kProjectionPartialBytesPerUs;
       }
       if (best_us < 0.0 || us < best_us) {
         best = {cost.tile, ranges, ranges > 1 ? per_range * slab : k};

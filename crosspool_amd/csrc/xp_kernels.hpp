@@ -186,28 +186,14 @@ struct RouterTopkArgs {
   int32_t softmax;  // 1: softmax scores, ties to the lower id; 0: sigmoid, ties to the higher id
   int32_t renormalize;
   int32_t round_to_logits;
-  // The bf16 projection's K-slice sums [slices, rows, experts] (fp32), or null: the TopK
-  // then adds each logit's slices in slice order, rounds the sum to bf16 once (the order and
-  // rounding of stream_reduce_kernel, whose launch this replaces) and stores it at
-  // logits_out (= logits) before selecting.
+  // The projection's K-slice sums [slices, rows, experts] (fp32), or null: the TopK then adds
+  // each logit's slices in slice order (for 16-bit logits rounding the sum once, the order
+  // and rounding of the reduction launch this replaces) and stores it at logits_out
+  // (= logits) before selecting.
   const float *partials;
-  uint16_t *logits_out;
+  void *logits_out;
   int32_t slices;
   int32_t payload;  // PayloadKind of 16-bit logits (logits_f32 == 0) and of their roundings
-};
-
-// Router logits[rows, experts] = x[rows, hidden] . w[experts, hidden] (w bf16 or fp32) as
-// fp32 sums, stored as fp32 or rounded to bf16.
-struct RouterLogitsArgs {
-  const uint16_t *x;
-  const void *w;
-  void *logits;
-  int64_t rows;
-  int64_t hidden;
-  int32_t experts;
-  int32_t weights_f32;
-  int32_t out_payload;  // logits stored in the payload dtype (else fp32)
-  int32_t payload;      // PayloadKind of x, of w unless weights_f32, and of payload logits
 };
 
 struct FinalizeRoutingArgs {
@@ -269,7 +255,6 @@ int moe_tile_rows(MoeTile tile);
 MoeTile choose_moe_tile(int64_t routes, int64_t experts);
 
 KernelLaunch make_router_topk(const RouterTopkArgs &args);
-KernelLaunch make_router_logits(const RouterLogitsArgs &args);
 KernelLaunch make_finalize_routing(const FinalizeRoutingArgs &args);
 KernelLaunch make_moe_sort(const MoeSortArgs &args);
 KernelLaunch make_moe_combine(const MoeCombineArgs &args);
@@ -325,8 +310,7 @@ struct ProjectionPlan {
   int64_t k_slice;
 };
 ProjectionPlan plan_projection(int64_t rows, int64_t n, int64_t k, int element_bytes, size_t scratch_bytes);
-// The most scratch plan_projection uses at 64, 128, ... and `capacity` rows (less scratch at
-// another row count only splits K less).
+// The most scratch plan_projection uses at any row count up to `capacity`.
 size_t projection_scratch_bytes(int64_t capacity, int64_t n, int64_t k, int element_bytes);
 
 // The projection and, for a K split, the launch that adds the ranges and applies the epilogue.

@@ -158,7 +158,7 @@ int xp_projection(const void *x, int64_t rows, int64_t k, const void *w, int64_t
 /* xp_projection with scratch for the fp32 sums of K ranges, so that a projection of few rows or
  * columns is spread over the whole device (GemmPlan's split-K workspace, linear.py:111-131).
  * `workspace` is 16-byte aligned and may be smaller than xp_projection_workspace_bytes (or null):
- * K is then split less.  The query is for any row count up to `rows`. */
+ * K is then split less.  The query covers every row count up to `rows`. */
 size_t xp_projection_workspace_bytes(int64_t rows, int64_t n, int64_t k, int dtype);
 int xp_projection_split(const void *x, int64_t rows, int64_t k, const void *w, int64_t n, const float *bias, void *out,
                         int dtype, const xp_activation_desc *activation, void *workspace, size_t workspace_bytes,

@@ -13,6 +13,8 @@ import pytest
 import torch
 
 from crosspool_amd import _native
+from crosspool_amd.ffn import RouterProjectionPrecision
+from crosspool_amd.moe import MoeRouterWeights, Router
 
 pytestmark = pytest.mark.gpu
 
@@ -98,3 +100,25 @@ def test_projection_keeps_infinities_and_nan_in_their_rows(device):
     got, expected = out[: rows * n].view(rows, n).float().cpu(), x.float().cpu() @ w.float().cpu().t() + bias.cpu()
     assert torch.equal(torch.isnan(got), torch.isnan(expected))
     assert torch.equal(torch.isinf(got), torch.isinf(expected)) and torch.equal(got[torch.isinf(got)], expected[torch.isinf(expected)])
+
+
+# The Router's fp32 logits: unsplit and K-split projections, capacities above the live rows,
+# 16-bit and fp32 weights, widths that are no multiple of 8.
+@pytest.mark.parametrize("precision", (RouterProjectionPrecision.FP32, RouterProjectionPrecision.FP32_LOGITS))
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))
+@pytest.mark.parametrize("rows,capacity,hidden,experts", ((1, 1, 40, 17), (9, 16, 2048, 128), (33, 66, 2048, 128), (65, 128, 1003, 130)))
+def test_router_fp32_logits(device, precision, dtype, rows, capacity, hidden, experts):
+    print(f"router {precision.name} {dtype} {rows}/{capacity}x{experts}x{hidden}", flush=True)
+    generator = torch.Generator(device=device).manual_seed(rows + hidden)
+    x = torch.randn((capacity, hidden), device=device, generator=generator).to(dtype)
+    weight_dtype = torch.float32 if precision is RouterProjectionPrecision.FP32 else dtype
+    w = torch.randn((experts, hidden), device=device, generator=generator).to(weight_dtype)
+    router = Router(row_capacity=capacity, hidden_size=hidden, routed_expert_count=experts, routed_topk=4,
+                    precision=precision, device=device, payload_dtype=dtype)
+    router.run_into(hidden_states=x, router_weights=MoeRouterWeights(w), rows=rows)
+    torch.cuda.synchronize()
+    _assert_within_bound(router.logits[:rows], x[:rows], w, None)
+    scores, order = torch.softmax(router.logits[:rows].cpu(), dim=1).sort(dim=1, descending=True, stable=True)
+    assert torch.equal(router.ids[:rows].cpu().long(), order[:, :4])
+    torch.testing.assert_close(router.weights[:rows].cpu(), scores[:, :4] / scores[:, :4].sum(1, keepdim=True), rtol=1e-5,
+                               atol=1e-6)
