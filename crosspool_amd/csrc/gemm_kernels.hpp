@@ -1591,13 +1591,19 @@ __device__ __forceinline__ void static_for(F &&f) {
 // J * (token tiles) = 32: the workgroups an XCD runs together then share the slabs of a few
 // token and weight tiles in its L2, and every weight tile is fetched by one XCD in one
 // round (Qwen3-8B gate_up at 2048 rows: 612 instead of 968 MB fetched per launch, same
-// time).  Otherwise the grid coordinates are used as they are (with 16 token tiles the
-// blocks took 3 % longer).  The results are wave-uniform; readfirstlane keeps them (and the
-// buffer resources built from them) in scalar registers.
+// time).  Weight tiles that do not split evenly are given out in runs of consecutive tiles of
+// such blocks instead (in grid order every token tile's copy of a weight tile was on another
+// XCD): gate_up of the Qwen3-32B TP shard (25 tiles of 256) at 2048 / 8192 rows 126 -> 119 and
+// 470 -> 461 us, of a hidden-1536 layer (70) at 896 rows on 128 x 256 tiles 67.6 -> 55.8,
+// Qwen3-4B down (10) at 4096 rows 207 -> 194; worst Qwen3-4B gate_up (76) at 2048 rows, 184 ->
+// 188.  With more than 8 token tiles and even weight tiles the grid coordinates are used as
+// they are (blocks took 3 % longer; runs 2 % less on 256 x 256 tiles, 5 % more on 256 x 128).
+// The results are wave-uniform; readfirstlane keeps them (and the buffer resources built from
+// them) in scalar registers.
 __device__ __forceinline__ void tile_coordinates(int &tn, int &tm) {
   const int nx = static_cast<int>(gridDim.x);
   const int ny = static_cast<int>(gridDim.y);
-  if (nx % 8 != 0 || ny > 8) {
+  if (nx % 8 == 0 && ny > 8) {
     tn = static_cast<int>(blockIdx.x);
     tm = static_cast<int>(blockIdx.y);
     return;
@@ -1605,13 +1611,29 @@ __device__ __forceinline__ void tile_coordinates(int &tn, int &tm) {
   const int linear = static_cast<int>(blockIdx.x) + nx * static_cast<int>(blockIdx.y);
   const int xcd = linear % 8;
   const int k = linear / 8;  // place in the XCD's dispatch order
-  const int per_xcd = nx / 8;
-  const int block_tiles = 32 / ny > per_xcd ? per_xcd : 32 / ny;
-  const int block = k / (block_tiles * ny);
-  const int rest = k - block * block_tiles * ny;
-  const int tiles = per_xcd - block * block_tiles < block_tiles ? per_xcd - block * block_tiles : block_tiles;
-  tm = __builtin_amdgcn_readfirstlane(rest / tiles);
-  tn = __builtin_amdgcn_readfirstlane(xcd + 8 * (block * block_tiles + rest % tiles));
+  if (nx % 8 == 0) {
+    const int per_xcd = nx / 8;
+    const int block_tiles = 32 / ny > per_xcd ? per_xcd : 32 / ny;
+    const int block = k / (block_tiles * ny);
+    const int rest = k - block * block_tiles * ny;
+    const int tiles = per_xcd - block * block_tiles < block_tiles ? per_xcd - block * block_tiles : block_tiles;
+    tm = __builtin_amdgcn_readfirstlane(rest / tiles);
+    tn = __builtin_amdgcn_readfirstlane(xcd + 8 * (block * block_tiles + rest % tiles));
+    return;
+  }
+  // Otherwise each XCD takes a run of consecutive tiles of one order over the whole grid:
+  // bands of 8 token tiles, and in a band blocks of J weight tiles x the band's token tiles.
+  const int total = nx * ny;
+  const int place = xcd * (total / 8) + (xcd < total % 8 ? xcd : total % 8) + k;
+  const int band = place / (8 * nx);
+  const int in_band = place - band * 8 * nx;
+  const int rows = ny - 8 * band < 8 ? ny - 8 * band : 8;
+  const int block_tiles = 32 / rows;
+  const int block = in_band / (block_tiles * rows);
+  const int rest = in_band - block * block_tiles * rows;
+  const int tiles = nx - block * block_tiles < block_tiles ? nx - block * block_tiles : block_tiles;
+  tm = __builtin_amdgcn_readfirstlane(8 * band + rest / tiles);
+  tn = __builtin_amdgcn_readfirstlane(block * block_tiles + rest % tiles);
 }
 
 // Weight tile tn and expert tile tm of a grouped projection's workgroup.  Every weight tile
