@@ -486,8 +486,11 @@ GemmLaunch make_gemm(const GemmArgs &args, int64_t capacity, bool gated, GemmCho
   GemmLaunch launches;
   KernelLaunch &kernel = launches.main;
   const bool f16 = args.payload == kPayloadF16;
-  auto tile_kernel = [&](int variant, bool stream) {
-    return f16 ? DenseKernels<F16Payload>::tile(gated, variant, stream) : DenseKernels<Bf16Payload>::tile(gated, variant, stream);
+  auto tile_kernel = [&](int variant) {
+    const WeightLoads loads = capacity > kTileShapes[variant].bm ? WeightLoads::Shared
+                              : args.k % kRotatedPitch == 0 && choice.k_split == 1 ? WeightLoads::StreamRotated
+                                                                                   : WeightLoads::Stream;
+    return f16 ? DenseKernels<F16Payload>::tile(gated, variant, loads) : DenseKernels<Bf16Payload>::tile(gated, variant, loads);
   };
   GemmArgs record = args;
   record.capacity = capacity;
@@ -558,16 +561,14 @@ GemmLaunch make_gemm(const GemmArgs &args, int64_t capacity, bool gated, GemmCho
       tail_record.n = choice.tail_columns;
       tail_record.w = args.w + n1 * args.k;
       tail_record.out = args.out + (gated ? n1 / 2 : n1);
-      const bool tail_stream = capacity <= other.bm;
-      launches.tail.func = tile_kernel(choice.tail_variant, tail_stream);
+      launches.tail.func = tile_kernel(choice.tail_variant);
       launches.tail.grid = dim3(static_cast<unsigned>((tail_record.n + other.bn - 1) / other.bn),
                                 static_cast<unsigned>((capacity + other.bm - 1) / other.bm), 1);
       launches.tail.block = dim3(static_cast<unsigned>(64 * other.waves), 1, 1);
       launches.tail.set_args(tail_record);
     }
     const TileShape &shape = kTileShapes[choice.variant];
-    const bool stream = capacity <= shape.bm;
-    kernel.func = tile_kernel(choice.variant, stream);
+    kernel.func = tile_kernel(choice.variant);
     kernel.grid = dim3(static_cast<unsigned>((n1 + shape.bn - 1) / shape.bn),
                        static_cast<unsigned>((capacity + shape.bm - 1) / shape.bm),
                        static_cast<unsigned>(choice.k_split));

@@ -67,23 +67,41 @@ const void *DenseKernels<P>::resident(bool gated, bool gather, int cpw, int grou
   return resident_kernel<kResidentGroups, false, false, P>(cpw);
 }
 
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool GATED, class P>
+const void *tile_kernel(WeightLoads loads) {
+  if (loads == WeightLoads::Shared) {
+    return kernel_address(&tile_gemm_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, GATED, false, false, P>);
+  }
+  if constexpr (BM <= kRotatedTileRows) {
+    if (loads == WeightLoads::StreamRotated) {
+      return kernel_address(&tile_gemm_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, GATED, false, true, P, false, true>);
+    }
+  }
+  return kernel_address(&tile_gemm_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, GATED, false, true, P>);
+}
+
 template <bool GATED, class P>
-const void *tile_kernel(int variant, bool stream) {
-  using Kernel = void (*)(GemmArgs);
-  static const Kernel table[][2] = {
-      {&tile_gemm_kernel<256, 256, 2, 4, 2, GATED, false, false, P>, &tile_gemm_kernel<256, 256, 2, 4, 2, GATED, false, true, P>},
-      {&tile_gemm_kernel<256, 128, 4, 2, 3, GATED, false, false, P>, &tile_gemm_kernel<256, 128, 4, 2, 3, GATED, false, true, P>},
-      {&tile_gemm_kernel<128, 128, 2, 2, 3, GATED, false, false, P>, &tile_gemm_kernel<128, 128, 2, 2, 3, GATED, false, true, P>},
-      {&tile_gemm_kernel<64, 128, 2, 2, 6, GATED, false, false, P>, &tile_gemm_kernel<64, 128, 2, 2, 6, GATED, false, true, P>},
-      {&tile_gemm_kernel<64, 64, 2, 1, 4, GATED, false, false, P>, &tile_gemm_kernel<64, 64, 2, 1, 4, GATED, false, true, P>},
-  };
-  static_assert(sizeof(table) / sizeof(table[0]) == kTileShapeCount, "one kernel per tile shape");
-  return kernel_address(table[variant][stream ? 1 : 0]);
+const void *tile_kernel(int variant, WeightLoads loads) {
+  static_assert(kTileShapeCount == 5, "one kernel per tile shape");
+  switch (variant) {
+    case 0:
+      return tile_kernel<256, 256, 2, 4, 2, GATED, P>(loads);
+    case 1:
+      return tile_kernel<256, 128, 4, 2, 3, GATED, P>(loads);
+    case 2:
+      return tile_kernel<128, 128, 2, 2, 3, GATED, P>(loads);
+    case 3:
+      return tile_kernel<64, 128, 2, 2, 6, GATED, P>(loads);
+    case 4:
+      return tile_kernel<64, 64, 2, 1, 4, GATED, P>(loads);
+    default:
+      return nullptr;
+  }
 }
 
 template <class P>
-const void *DenseKernels<P>::tile(bool gated, int variant, bool stream) {
-  return gated ? tile_kernel<true, P>(variant, stream) : tile_kernel<false, P>(variant, stream);
+const void *DenseKernels<P>::tile(bool gated, int variant, WeightLoads loads) {
+  return gated ? tile_kernel<true, P>(variant, loads) : tile_kernel<false, P>(variant, loads);
 }
 
 }  // namespace xp

@@ -1852,7 +1852,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs &a, const f32x16 (&
 // range each workgroup writes the fp32 partial tile of its range and
 // stream_reduce_kernel, launched next, adds the ranges in order and applies the epilogue.
 template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, bool GATED, bool GROUPED = false,
-          bool STREAM_WEIGHTS = GROUPED, class PAYLOAD = Bf16Payload, bool EXTENDED = false>
+          bool STREAM_WEIGHTS = GROUPED, class PAYLOAD = Bf16Payload, bool EXTENDED = false, bool ROTATE = false>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_gemm_kernel(GemmArgs a) {
   constexpr int BK = 64;
   constexpr int WAVES = WAVES_M * WAVES_N;
@@ -1976,12 +1976,28 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_gemm_kernel(GemmA
       return p;
     }
   };
+  // The chooser never makes an empty K range, so every workgroup runs at least one slab.
+  const int64_t ktiles = (k_end - k_begin + BK - 1) / BK;
+  // ROTATE: the workgroups of a launch start at different slabs of K.  Weight rows a whole
+  // number of 8 KB apart put the slabs that workgroups walking K from column 0 stream at one
+  // time on the same few memory channels; with one token tile the weights come straight from
+  // HBM, once.  Qwen3-8B gate_up (K = 4096) at 32 / 45 / 64 rows on 64 x 128 tiles 43.6 / 44.2 /
+  // 42.1 -> 34.9 / 36.3 / 37.9 us (5.6 TB/s), at 128 on 128 x 128 50.0 -> 45.6.  Other row
+  // pitches gain nothing, and neither do 256-row tiles or several token tiles, whose workgroups
+  // share the slabs they stream in L2 (2048 rows: 309 -> 315 us).
+  [[maybe_unused]] const int rotation =
+      ROTATE ? __builtin_amdgcn_readfirstlane(tn * 7 % static_cast<int>(ktiles)) : 0;
   // Slab kt of this workgroup's K range.  Slabs at or past the range end (the prologue of
   // a short range, the refills after the last slab) load zeros without memory traffic.
   // PART selects the A loads (1), the B loads (2) or both (3).
   auto issue_part = [&](int64_t kt, int stage, auto part) XP_INLINE {
     constexpr int PART = decltype(part)::value;
-    const int64_t k_pos = k_begin + kt * BK;
+    int64_t slab = kt;
+    if constexpr (ROTATE) {
+      slab = kt + rotation < ktiles ? kt + rotation : kt + rotation - ktiles;
+      slab = kt < ktiles ? slab : ktiles;
+    }
+    const int64_t k_pos = k_begin + slab * BK;
     const uint32_t k_bytes = static_cast<uint32_t>(k_pos * 2);
     // 16-byte chunks of this slab that lie inside the range (8 except in a ragged last slab).
     const int64_t chunks_left = (k_end - k_pos) >> 3;
@@ -2119,8 +2135,6 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void tile_gemm_kernel(GemmA
   if (a.scatter_slots != nullptr && a.k_split == 1) {
     load_row_meta<WTM>(a, m0, row_end, wm, meta);
   }
-  // The chooser never makes an empty K range, so every workgroup runs at least one slab.
-  const int64_t ktiles = (k_end - k_begin + BK - 1) / BK;
   // Prologue: slabs 0 .. STAGES-1 in flight, wait for slab 0, read its first fragments.
   if (loading_wave) {
 #pragma unroll

@@ -58,6 +58,15 @@ constexpr int kNarrowDecodeTile = 4;  // 64 x 64
 // chunk counts that do not divide into its groups) 122.4 / 217.0 / 238.7.
 constexpr int kGroupedSplitDepth = 2;
 
+// How a tile launch loads its weights, each its own instantiation (a per-load branch on an
+// argument cost the loading waves ~2 % at 2048 rows).  Stream: the grid has one token tile, so
+// each weight tile has one reader and its loads carry the nontemporal hint.  StreamRotated: the
+// same from another slab of K in each workgroup, for weight rows a multiple of 8 KB apart (the
+// kernel's ROTATE).
+enum class WeightLoads : int { Shared = 0, Stream = 1, StreamRotated = 2 };
+constexpr int kRotatedTileRows = 128;
+constexpr int64_t kRotatedPitch = 4096;  // columns
+
 template <class P>
 struct DenseKernels {
   // The split kernel for `groups` token groups of 8 (1 or 2); the fused gather takes one.
@@ -72,10 +81,7 @@ struct DenseKernels {
   // Null for a combination without an instantiation (four groups serve gate_up with the
   // gather fused only).
   static const void *resident(bool gated, bool gather, int cpw, int groups);
-  // STREAM: the grid has one token tile, so each weight tile has one reader and its loads
-  // carry the nontemporal hint (a compile-time policy: a per-load branch on an argument cost
-  // the loading waves ~2 % at 2048 rows).
-  static const void *tile(bool gated, int variant, bool stream);
+  static const void *tile(bool gated, int variant, WeightLoads loads);
 };
 
 template <class P>
