@@ -345,6 +345,124 @@ GemmChoice choose_gemm(int64_t capacity, int64_t n, int64_t k, bool gated, bool 
   return choice;
 }
 
+// Tile, K split or column split of a Dense step's projection above kStepMinRows rows, from a
+// model of one launch in microseconds: whole rounds of one tile per CU, each at the shape's
+// full rate, and a last round whose slabs go the faster the fewer CUs it fills (the chip
+// clocks higher and its L2s have fewer readers); the weights' stream adds to it, since a round's
+// tiles wait for the same lines; a K split adds its reduction and its sums' traffic.  A
+// column split is two such launches.
+// Fitted (log least squares) to 9400 forced choices on MI355X: Qwen3 0.6B / 1.7B / 4B / 8B, a
+// hidden-1536 layer and the Qwen3-32B TP shard, both projections, 26 row counts from 65 to 4096,
+// every shape and 1 to 16 K ranges, weights streamed from HBM: mean error 6.1 %, and its picks
+// sum to 0.6 % above the fastest measured single launch of each.  The column splits it prices
+// were measured too (183 of them); they cost 11 % more than two modelled launches plus
+// kStepTailUs.  The choice for the template's capacity stays unless the model prices another
+// kStepGain below it, about the model's error: over the same sweep that loses against it in one
+// case (3.9 %) and sums to 1 % above the best, where choose_gemm's choices (which know neither
+// 192 x 256 and 128 x 256 tiles nor K splits that are no power of two) sum to 6 % above.
+struct StepTile {
+  int variant;
+  double slab_us;   // per 64 columns of a round, however full
+  double fill_us;   // the same, times the share of the CUs the round fills
+  double tile_us;   // prologue and epilogue of a round
+};
+constexpr StepTile kStepTiles[] = {
+    {0, 1.091, 0.203, 4.50},  // 256 x 256
+    {1, 0.544, 0.156, 3.21},  // 256 x 128
+    {2, 0.412, 0.073, 2.97},  // 128 x 128
+    {3, 0.272, 0.082, 2.35},  // 64 x 128
+    {5, 0.999, 0.141, 3.62},  // 192 x 256
+    {6, 0.612, 0.148, 3.24},  // 128 x 256
+};
+constexpr int64_t kStepMinRows = 65;
+constexpr int64_t kStepSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
+constexpr int64_t kStepMinSlabs = 3;  // per K range
+constexpr double kStepLaunchUs = 2.42;
+constexpr double kStepReduceUs = 4.21;
+constexpr double kStepPartialBytesPerUs = 7.76e6;
+constexpr double kStepWeightBytesPerUs = 16.7e6;
+constexpr double kStepTailUs = 5.6;
+constexpr double kStepTailScale = 1.11;
+constexpr double kStepGain = 0.10;
+
+// Compute time of one launch of `weight_tiles` x the token tiles x `splits` workgroups.
+double step_compute_us(const StepTile &tile, int64_t capacity, int64_t n, int64_t slabs, int64_t splits) {
+  const TileShape &shape = kTileShapes[tile.variant];
+  const int64_t workgroups = (capacity + shape.bm - 1) / shape.bm * ((n + shape.bn - 1) / shape.bn) * splits;
+  const int64_t rounds = workgroups / kComputeUnits;
+  const double rest = static_cast<double>(workgroups - rounds * kComputeUnits) / kComputeUnits;
+  const double columns = static_cast<double>(slabs);
+  double us = static_cast<double>(rounds) * (columns * (tile.slab_us + tile.fill_us) + tile.tile_us);
+  if (rest > 0.0) {
+    us += columns * (tile.slab_us + tile.fill_us * rest) + tile.tile_us;
+  }
+  return us;
+}
+
+// The model's time of a tile choice at `rows` rows, or -1 where it has no figures (64 x 64).
+double step_us(const GemmChoice &choice, int64_t rows, int64_t n, int64_t k, double tail_scale = kStepTailScale) {
+  const StepTile *main = nullptr;
+  const StepTile *tail = nullptr;
+  for (const StepTile &tile : kStepTiles) {
+    main = tile.variant == choice.variant ? &tile : main;
+    tail = tile.variant == choice.tail_variant ? &tile : tail;
+  }
+  if (main == nullptr || (choice.tail_columns > 0 && tail == nullptr)) {
+    return -1.0;
+  }
+  const int64_t slabs = (choice.k_slice + 63) / 64;
+  double us = kStepLaunchUs + step_compute_us(*main, rows, n - choice.tail_columns, slabs, choice.k_split) +
+              2.0 * static_cast<double>(n) * static_cast<double>(k) / kStepWeightBytesPerUs;
+  if (choice.k_split > 1) {
+    us += kStepReduceUs + 8.0 * static_cast<double>(choice.k_split * rows * n) / kStepPartialBytesPerUs;
+  }
+  if (choice.tail_columns > 0) {
+    us = tail_scale * (us + step_compute_us(*tail, rows, choice.tail_columns, slabs, 1)) + kStepTailUs;
+  }
+  return us;
+}
+
+GemmChoice choose_step_tile(const GemmChoice &base, int64_t rows, int64_t n, int64_t k) {
+  const int64_t slabs = (k + 63) / 64;
+  GemmChoice best = base;
+  const double base_us = step_us(base, rows, n, k, 1.0);  // a column split's lower price
+  if (base_us < 0.0) {
+    return base;
+  }
+  double best_us = base_us * (1.0 - kStepGain);
+  auto consider = [&](const GemmChoice &choice) {
+    const double us = step_us(choice, rows, n, k);
+    if (us < best_us) {
+      best = choice;
+      best_us = us;
+    }
+  };
+  for (const StepTile &tile : kStepTiles) {
+    for (const int64_t splits : kStepSplits) {
+      const int64_t per_range = (slabs + splits - 1) / splits;
+      if (splits == 1 || (per_range >= kStepMinSlabs && (splits - 1) * per_range < slabs)) {  // none empty
+        consider({GemmKind::Tile, tile.variant, splits > 1 ? per_range * 64 : k, splits});
+      }
+    }
+    // A first launch of nearly whole rounds, and the remaining columns in a second one.
+    const TileShape &shape = kTileShapes[tile.variant];
+    const int64_t token_tiles = (rows + shape.bm - 1) / shape.bm;
+    for (int64_t weight_tiles = 1; weight_tiles * shape.bn < n; ++weight_tiles) {
+      const int64_t partial = token_tiles * weight_tiles % kComputeUnits;
+      if (token_tiles * weight_tiles < kComputeUnits * 3 / 4 || (partial != 0 && partial < kComputeUnits * 11 / 12)) {
+        continue;
+      }
+      GemmChoice choice{GemmKind::Tile, tile.variant, k, 1};
+      choice.tail_columns = n - weight_tiles * shape.bn;
+      for (const StepTile &other : kStepTiles) {
+        choice.tail_variant = other.variant;
+        consider(choice);
+      }
+    }
+  }
+  return best;
+}
+
 // The fused gather's prologue (slot list, full-row sums of squares, staging) runs in every
 // workgroup, so the fused gate_up takes the fewest K slices that fit LDS (measured: 4
 // slices of Qwen3-8B gate_up took 47 + 5 us against 38 us for one).  Up to kSplitMaxRows
@@ -418,6 +536,10 @@ GemmChoice choose_dense_gate_up(int64_t capacity, int64_t n, int64_t k, bool &fu
     return separate;
   }
   return fused_choice;
+}
+
+GemmChoice refine_dense_choice(const GemmChoice &base, int64_t rows, int64_t n, int64_t k) {
+  return base.kind == GemmKind::Tile && rows >= kStepMinRows ? choose_step_tile(base, rows, n, k) : base;
 }
 
 bool split_gather_fusable(int64_t capacity, int64_t n, int64_t k) {

@@ -82,7 +82,7 @@ const void *tile_kernel(WeightLoads loads) {
 
 template <bool GATED, class P>
 const void *tile_kernel(int variant, WeightLoads loads) {
-  static_assert(kTileShapeCount == 5, "one kernel per tile shape");
+  static_assert(kTileShapeCount == 7, "one kernel per tile shape");
   switch (variant) {
     case 0:
       return tile_kernel<256, 256, 2, 4, 2, GATED, P>(loads);
@@ -94,6 +94,10 @@ const void *tile_kernel(int variant, WeightLoads loads) {
       return tile_kernel<64, 128, 2, 2, 6, GATED, P>(loads);
     case 4:
       return tile_kernel<64, 64, 2, 1, 4, GATED, P>(loads);
+    case 5:
+      return tile_kernel<192, 256, 2, 4, 2, GATED, P>(loads);
+    case 6:
+      return tile_kernel<128, 256, 2, 4, 3, GATED, P>(loads);
     default:
       return nullptr;
   }

@@ -37,6 +37,8 @@ constexpr TileShape kTileShapes[] = {
     {128, 128, 4, 3, 3.4e6},
     {64, 128, 4, 6, 2.4e6},
     {64, 64, 2, 4, 1.2e6},
+    {192, 256, 8, 2, 4.5e6},
+    {128, 256, 8, 3, 4.2e6},
 };
 constexpr int kTileShapeCount = sizeof(kTileShapes) / sizeof(kTileShapes[0]);
 // The cost model ranks the first four shapes.  The 64 x 64 gated tile (two waves, four

@@ -57,11 +57,60 @@ constexpr size_t kRegionAlignment = 16;
 
 size_t align_up(size_t value, size_t alignment) { return (value + alignment - 1) / alignment * alignment; }
 
-// Workspace regions of one Dense step at `capacity`: gathered batch [capacity, hidden],
-// then the activated intermediate [capacity, intermediate], each 16-byte aligned; then,
-// when a projection at this capacity splits K across workgroups (sliced stream or split
-// tile kernel), the fp32 partial sums of its K ranges (256-byte aligned, gate_up's then
-// down's).
+// Kernel choices of a Dense step whose grids serve up to `rows` rows.
+struct DensePlan {
+  int64_t rows;
+  GemmChoice gate_up;
+  GemmChoice down;
+  bool fused;  // the gather runs inside gate_up
+};
+
+// The choices for a capacity, before they are refined for a number of live rows.
+DensePlan plan_dense_capacity(int64_t capacity, int64_t hidden, int64_t intermediate) {
+  DensePlan plan{};
+  plan.rows = capacity;
+  plan.gate_up = choose_dense_gate_up(capacity, 2 * intermediate, hidden, plan.fused);
+  plan.down = choose_gemm(capacity, hidden, intermediate, false);
+  return plan;
+}
+
+DensePlan refine_plan(const DensePlan &base, int64_t rows, int64_t hidden, int64_t intermediate) {
+  DensePlan plan = base;
+  plan.rows = rows;
+  plan.gate_up = refine_dense_choice(base.gate_up, rows, 2 * intermediate, hidden);
+  plan.down = refine_dense_choice(base.down, rows, hidden, intermediate);
+  return plan;
+}
+
+// A template of more than 64 rows holds a plan per kPlanSteps-th of its capacity (at least 64
+// rows apart, one token tile), and a replay takes the smallest that covers its live rows: the
+// tile shapes, K splits and column splits then suit what runs rather than up to twice as
+// many rows.  Layers at 517 rows of a 1024-row template: Qwen3-4B 158 -> 117 us, 8B 222 -> 184,
+// 1.7B 75 -> 61, the 32B TP shard 93 -> 79; over 23 row counts from 100 to 4000 and six shapes
+// 1.07 times as fast.
+constexpr int64_t kPlanRowStep = 64;
+constexpr int64_t kPlanSteps = 16;
+
+int64_t plan_row_step(int64_t capacity) {
+  const int64_t unit = kPlanSteps * kPlanRowStep;
+  return (capacity + unit - 1) / unit * kPlanRowStep;
+}
+
+std::vector<DensePlan> plan_dense_template(int64_t capacity, int64_t hidden, int64_t intermediate) {
+  std::vector<DensePlan> plans;
+  const DensePlan base = plan_dense_capacity(capacity, hidden, intermediate);
+  const int64_t step = plan_row_step(capacity);
+  for (int64_t rows = step; rows < capacity; rows += step) {
+    plans.push_back(refine_plan(base, rows, hidden, intermediate));
+  }
+  plans.push_back(refine_plan(base, capacity, hidden, intermediate));
+  return plans;
+}
+
+// Workspace regions of a Dense step at `capacity`: gathered batch [capacity, hidden], then the
+// activated intermediate [capacity, intermediate], each 16-byte aligned; then, when a
+// projection of one of the plans splits K across workgroups (sliced stream or split tile
+// kernel), the fp32 partial sums of its K ranges (256-byte aligned, gate_up's then down's).
 struct DenseWorkspace {
   size_t batch_offset;
   size_t activated_offset;
@@ -70,16 +119,19 @@ struct DenseWorkspace {
   size_t bytes;
 };
 
-DenseWorkspace dense_workspace(int64_t capacity, int64_t hidden, int64_t intermediate) {
+DenseWorkspace dense_workspace(int64_t capacity, int64_t hidden, int64_t intermediate, const DensePlan *plans,
+                               size_t plan_count) {
   DenseWorkspace layout{};
   layout.batch_offset = 0;
   layout.activated_offset = align_up(static_cast<size_t>(capacity * hidden) * 2, kRegionAlignment);
   size_t cursor = layout.activated_offset + static_cast<size_t>(capacity * intermediate) * 2;
-  bool fused = false;
-  const size_t gate_up = gemm_scratch_bytes(choose_dense_gate_up(capacity, 2 * intermediate, hidden, fused),
-                                            capacity, 2 * intermediate, hidden);
-  const size_t down = gemm_scratch_bytes(choose_gemm(capacity, hidden, intermediate, false), capacity, hidden,
-                                         intermediate);
+  size_t gate_up = 0;
+  size_t down = 0;
+  for (size_t index = 0; index < plan_count; ++index) {
+    const DensePlan &plan = plans[index];
+    gate_up = std::max(gate_up, gemm_scratch_bytes(plan.gate_up, plan.rows, 2 * intermediate, hidden));
+    down = std::max(down, gemm_scratch_bytes(plan.down, plan.rows, hidden, intermediate));
+  }
   if (gate_up + down > 0) {
     cursor = align_up(cursor, 256);
     layout.gate_up_partials_offset = cursor;
@@ -89,6 +141,12 @@ DenseWorkspace dense_workspace(int64_t capacity, int64_t hidden, int64_t interme
   }
   layout.bytes = cursor;
   return layout;
+}
+
+// The workspace of a template.
+DenseWorkspace dense_workspace(int64_t capacity, int64_t hidden, int64_t intermediate) {
+  const std::vector<DensePlan> plans = plan_dense_template(capacity, hidden, intermediate);
+  return dense_workspace(capacity, hidden, intermediate, plans.data(), plans.size());
 }
 
 // Buffer resources are 32-bit.  The split and stream kernels address a whole weight matrix
@@ -128,8 +186,8 @@ int payload_kind(int dtype, int32_t &out) {
 // The kernels of one mailbox step, for a given capacity: gather (+ RMSNorm), gate_up
 // with the gated SiLU fused (+ its K-slice reduction), down with the scatter fused (+ its
 // reduction).  At decode sizes the gather is fused into gate_up and has no launch of its
-// own.  The sequence depends only on the capacity and geometry, so a template's node list
-// matches every replay's.
+// own.  The sequence depends only on the plan and geometry, so the nodes of a plan's graph
+// match every replay on it.
 struct DenseLaunches {
   KernelLaunch gather;
   GemmLaunch gate_up;
@@ -182,14 +240,13 @@ struct DenseBinding {
   int32_t payload;  // PayloadKind
 };
 
-DenseLaunches make_dense_launches(const DenseBinding &b, int64_t capacity) {
-  const DenseWorkspace layout = dense_workspace(capacity, b.hidden, b.intermediate);
+DenseLaunches make_dense_launches(const DenseBinding &b, const DenseWorkspace &layout, const DensePlan &plan) {
+  const int64_t capacity = plan.rows;
+  const bool fused = plan.fused;
   uint16_t *batch = reinterpret_cast<uint16_t *>(b.workspace + layout.batch_offset);
   uint16_t *activated = reinterpret_cast<uint16_t *>(b.workspace + layout.activated_offset);
   DenseLaunches launches;
 
-  bool fused = false;
-  const GemmChoice gate_up_choice = choose_dense_gate_up(capacity, 2 * b.intermediate, b.hidden, fused);
   if (!fused) {
     GatherArgs gather{};
     gather.pool = b.pool_in;
@@ -226,7 +283,7 @@ DenseLaunches make_dense_launches(const DenseBinding &b, int64_t capacity) {
     gate_up.pool_rows = b.pool_rows;
     gate_up.eps = b.eps;
   }
-  launches.gate_up = make_gemm(gate_up, capacity, true, gate_up_choice, fused);
+  launches.gate_up = make_gemm(gate_up, capacity, true, plan.gate_up, fused);
 
   GemmArgs down{};
   down.x = activated;
@@ -242,7 +299,7 @@ DenseLaunches make_dense_launches(const DenseBinding &b, int64_t capacity) {
   down.act = default_activation();
   down.payload = b.payload;
   down.partials = reinterpret_cast<float *>(b.workspace + layout.down_partials_offset);
-  launches.down = make_gemm(down, capacity, false, choose_gemm(capacity, down.n, down.k, false));
+  launches.down = make_gemm(down, capacity, false, plan.down);
   return launches;
 }
 
@@ -316,13 +373,8 @@ struct xp_agent {
   int live_lanes = 0;
 };
 
-struct Template {
-  int kind = XP_LAYER_DENSE;
-  int64_t hidden = 0;
-  int64_t intermediate = 0;
-  int32_t payload = kPayloadBf16;
-  int64_t capacity = 0;
-  xp_moe_layer_desc moe{};  // MoE templates: the signature they were captured for
+// The instantiated hipGraph of one plan.
+struct TemplateGraph {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   hipGraphNode_t nodes[kMaxTemplateKernels] = {};
@@ -330,6 +382,20 @@ struct Template {
   // Argument records last bound to each node: a replay rebinds only the nodes whose
   // record changed.
   KernelLaunch bound[kMaxTemplateKernels];
+};
+
+struct Template {
+  int kind = XP_LAYER_DENSE;
+  int64_t hidden = 0;
+  int64_t intermediate = 0;
+  int32_t payload = kPayloadBf16;
+  int64_t capacity = 0;
+  xp_moe_layer_desc moe{};  // MoE templates: the signature they were captured for
+  std::vector<DensePlan> plans;  // Dense templates, by rows; the last serves the capacity
+  DenseWorkspace layout{};
+  // One per plan (MoE templates: one).  The capacity's is instantiated at capture, the others
+  // at their first replay through graph dispatch.
+  std::vector<std::unique_ptr<TemplateGraph>> graphs;
 };
 
 struct xp_lane {
@@ -994,7 +1060,7 @@ bool valid_arena(xp_transport_t transport, int arena) {
 }
 
 
-void destroy_template(Template &t) {
+void destroy_graph(TemplateGraph &t) {
   if (t.exec != nullptr) {
     (void)hipGraphExecDestroy(t.exec);
     t.exec = nullptr;
@@ -1005,8 +1071,16 @@ void destroy_template(Template &t) {
   }
 }
 
-StepChain dense_chain(const DenseBinding &binding, int64_t capacity) {
-  const DenseLaunches launches = make_dense_launches(binding, capacity);
+void destroy_template(Template &t) {
+  for (auto &graph : t.graphs) {
+    if (graph != nullptr) {
+      destroy_graph(*graph);
+    }
+  }
+}
+
+StepChain dense_chain(const DenseBinding &binding, const DenseWorkspace &layout, const DensePlan &plan) {
+  const DenseLaunches launches = make_dense_launches(binding, layout, plan);
   const KernelLaunch *kernels[kMaxStepKernels];
   const int count = launches.chain(kernels);
   StepChain chain;
@@ -1017,12 +1091,14 @@ StepChain dense_chain(const DenseBinding &binding, int64_t capacity) {
   return chain;
 }
 
-// Build and instantiate a template's hipGraph: one kernel node per chain entry, each
-// depending on the previous one.
-int instantiate_template(Template &t, const StepChain &chain) {
+// Build and instantiate a plan's hipGraph: one kernel node per chain entry, each depending on
+// the previous one.
+int instantiate_graph(std::unique_ptr<TemplateGraph> &out, const StepChain &chain) {
   if (!chain.usable) {
     return fail(XP_ERROR_INVALID_ARGUMENT, kUnusableChoice);
   }
+  auto owned = std::make_unique<TemplateGraph>();
+  TemplateGraph &t = *owned;
   XP_HIP_CHECK(hipGraphCreate(&t.graph, 0));
   t.node_count = chain.count;
   for (int index = 0; index < chain.count; ++index) {
@@ -1030,7 +1106,7 @@ int instantiate_template(Template &t, const StepChain &chain) {
     if (kernel.shmem > 64 * 1024) {
       const hipError_t enabled = enable_large_lds(kernel.func);
       if (enabled != hipSuccess) {
-        destroy_template(t);
+        destroy_graph(t);
         return fail(XP_ERROR_HIP, std::string("enabling dynamic LDS above 64 KB failed: ") + hipGetErrorString(enabled));
       }
     }
@@ -1039,16 +1115,17 @@ int instantiate_template(Template &t, const StepChain &chain) {
     const hipGraphNode_t *dependencies = index == 0 ? nullptr : &t.nodes[index - 1];
     const hipError_t added = hipGraphAddKernelNode(&t.nodes[index], t.graph, dependencies, index == 0 ? 0 : 1, &node);
     if (added != hipSuccess) {
-      destroy_template(t);
+      destroy_graph(t);
       return fail(XP_ERROR_HIP, std::string("hipGraphAddKernelNode failed: ") + hipGetErrorString(added));
     }
     t.bound[index] = kernel;
   }
   const hipError_t instantiated = hipGraphInstantiate(&t.exec, t.graph, nullptr, nullptr, 0);
   if (instantiated != hipSuccess) {
-    destroy_template(t);
+    destroy_graph(t);
     return fail(XP_ERROR_HIP, std::string("hipGraphInstantiate failed: ") + hipGetErrorString(instantiated));
   }
+  out = std::move(owned);
   return XP_OK;
 }
 
@@ -1063,13 +1140,10 @@ void insert_template(xp_lane *lane, std::unique_ptr<Template> t) {
 }
 
 // Launch a replay's chain: directly on the stream, or (graph dispatch) by rebinding the
-// template's nodes whose argument record changed and launching its graph.
-int run_chain(xp_lane *lane, Template &t, const StepChain &chain, hipStream_t target) {
+// nodes of its plan's graph whose argument record changed and launching that graph.
+int run_chain(xp_lane *lane, std::unique_ptr<TemplateGraph> &graph, const StepChain &chain, hipStream_t target) {
   if (!chain.usable) {
     return fail(XP_ERROR_INVALID_ARGUMENT, kUnusableChoice);
-  }
-  if (chain.count != t.node_count) {
-    return fail(XP_ERROR_STATE, "replay kernel sequence differs from the captured template");
   }
   // Under an outer stream capture (a caller recording its decode step as a graph) the
   // kernels are launched directly, so that they become nodes of the caller's graph rather
@@ -1083,6 +1157,15 @@ int run_chain(xp_lane *lane, Template &t, const StepChain &chain, hipStream_t ta
       XP_HIP_CHECK(launch(chain.kernels[index], target));
     }
     return XP_OK;
+  }
+  if (graph == nullptr) {
+    if (const int status = instantiate_graph(graph, chain); status != XP_OK) {
+      return status;
+    }
+  }
+  TemplateGraph &t = *graph;
+  if (chain.count != t.node_count) {
+    return fail(XP_ERROR_STATE, "replay kernel sequence differs from the captured template");
   }
   for (int index = 0; index < chain.count; ++index) {
     const KernelLaunch &kernel = chain.kernels[index];
@@ -1455,9 +1538,23 @@ int dense_step_checks(const void *pool_in, const void *pool_out, int64_t pool_ro
   return XP_OK;
 }
 
+// The plan of a step at exactly `rows` rows that fits a workspace of `bytes`: the refined one,
+// else the capacity's own (less scratch).  `needed`: the least bytes that would have served.
+bool plan_dense_step(int64_t rows, int64_t hidden, int64_t intermediate, size_t bytes, DensePlan &plan, size_t &needed) {
+  const DensePlan base = plan_dense_capacity(rows, hidden, intermediate);
+  plan = refine_plan(base, rows, hidden, intermediate);
+  needed = dense_workspace(rows, hidden, intermediate, &plan, 1).bytes;
+  if (needed > bytes) {
+    plan = base;
+    needed = std::min(needed, dense_workspace(rows, hidden, intermediate, &plan, 1).bytes);
+  }
+  return dense_workspace(rows, hidden, intermediate, &plan, 1).bytes <= bytes;
+}
+
 int run_dense_step(const void *pool_in, void *pool_out, int64_t pool_rows, const int32_t *slots, int64_t rows,
                    int64_t hidden, int64_t intermediate, const void *w_gate_up, const void *w_down,
-                   const void *norm_weight, float eps, void *workspace, uint32_t *fault_word, xp_stream_t stream) {
+                   const void *norm_weight, float eps, void *workspace, uint32_t *fault_word, const DensePlan &plan,
+                   xp_stream_t stream) {
   DenseBinding binding{};
   binding.pool_in = static_cast<const uint16_t *>(pool_in);
   binding.pool_out = static_cast<uint16_t *>(pool_out);
@@ -1472,7 +1569,8 @@ int run_dense_step(const void *pool_in, void *pool_out, int64_t pool_rows, const
   binding.eps = eps;
   binding.workspace = static_cast<uint8_t *>(workspace);
   binding.fault = fault_word;
-  const DenseLaunches launches = make_dense_launches(binding, rows);
+  const DenseLaunches launches =
+      make_dense_launches(binding, dense_workspace(rows, hidden, intermediate, &plan, 1), plan);
   XP_REQUIRE(launches.usable(), kUnusableChoice);
   const KernelLaunch *chain[kMaxStepKernels];
   const int count = launches.chain(chain);
@@ -1495,10 +1593,12 @@ int xp_dense_step(const void *pool_in, void *pool_out, int64_t pool_rows, const 
   }
   XP_REQUIRE(workspace != nullptr, "dense step pointers must be non-null");
   XP_REQUIRE(aligned16(workspace), "dense step operands must be 16-byte aligned");
-  XP_REQUIRE(workspace_bytes >= dense_workspace(rows, hidden, intermediate).bytes,
+  DensePlan plan{};
+  size_t needed = 0;
+  XP_REQUIRE(plan_dense_step(rows, hidden, intermediate, workspace_bytes, plan, needed),
              "workspace is smaller than xp_dense_workspace_bytes(rows, hidden, intermediate)");
   return run_dense_step(pool_in, pool_out, pool_rows, slots, rows, hidden, intermediate, w_gate_up, w_down,
-                        norm_weight, eps, workspace, fault_word, stream);
+                        norm_weight, eps, workspace, fault_word, plan, stream);
 }
 
 // Workspace of xp_dense_step_static: a static device array, so that the step allocates
@@ -1542,8 +1642,9 @@ int xp_dense_step_static(const void *pool_in, void *pool_out, int64_t pool_rows,
       status != XP_OK || rows == 0) {
     return status;
   }
-  const size_t needed = dense_workspace(rows, hidden, intermediate).bytes;
-  if (needed > kStaticScratchBytes) {
+  DensePlan plan{};
+  size_t needed = 0;
+  if (!plan_dense_step(rows, hidden, intermediate, kStaticScratchBytes, plan, needed)) {
     return fail(XP_ERROR_CAPACITY, "dense step needs " + std::to_string(needed) +
                                        " bytes of workspace, more than the static scratch holds (" +
                                        std::to_string(kStaticScratchBytes) + " bytes); use xp_dense_step");
@@ -1553,7 +1654,7 @@ int xp_dense_step_static(const void *pool_in, void *pool_out, int64_t pool_rows,
     return status;
   }
   return run_dense_step(pool_in, pool_out, pool_rows, slots, rows, hidden, intermediate, w_gate_up, w_down,
-                        norm_weight, eps, workspace, fault_word, stream);
+                        norm_weight, eps, workspace, fault_word, plan, stream);
 }
 
 size_t xp_gemm_variant(int64_t capacity, int64_t n, int64_t k, int gated, char *buffer, size_t size) {
@@ -1570,7 +1671,8 @@ size_t xp_dense_gate_up_variant(int64_t capacity, int64_t hidden, int64_t interm
   std::string name;
   if (capacity > 0 && hidden > 0 && intermediate > 0) {
     bool fused = false;
-    const GemmChoice choice = choose_dense_gate_up(capacity, 2 * intermediate, hidden, fused);
+    const GemmChoice choice = refine_dense_choice(choose_dense_gate_up(capacity, 2 * intermediate, hidden, fused),
+                                                  capacity, 2 * intermediate, hidden);
     name = gemm_name(choice, true) + (fused ? "+gather" : "");  // SplitGathered names itself
   }
   if (buffer != nullptr && size > 0) {
@@ -1769,7 +1871,11 @@ int xp_template_capture(xp_lane_t lane, int64_t hidden, int64_t intermediate, in
   t->intermediate = intermediate;
   t->payload = payload;
   t->capacity = capacity;
-  if (const int status = instantiate_template(*t, dense_chain(binding, capacity)); status != XP_OK) {
+  t->plans = plan_dense_template(capacity, hidden, intermediate);
+  t->layout = dense_workspace(capacity, hidden, intermediate, t->plans.data(), t->plans.size());
+  t->graphs.resize(t->plans.size());
+  if (const int status = instantiate_graph(t->graphs.back(), dense_chain(binding, t->layout, t->plans.back()));
+      status != XP_OK) {
     return status;
   }
   insert_template(lane, std::move(t));
@@ -1851,7 +1957,7 @@ int xp_replay(xp_lane_t lane, int instance_index, int layer_ordinal, int64_t row
     if (const int status = make_moe_step(layer, binding, selected->capacity, chain); status != XP_OK) {
       return status;
     }
-    return run_chain(lane, *selected, chain, target);
+    return run_chain(lane, selected->graphs.front(), chain, target);
   }
   DenseBinding binding{};
   binding.pool_in = static_cast<const uint16_t *>(pool_in);
@@ -1868,7 +1974,11 @@ int xp_replay(xp_lane_t lane, int instance_index, int layer_ordinal, int64_t row
   binding.workspace = lane->workspace;
   binding.fault = lane->fault;
   binding.payload = layer.payload;
-  return run_chain(lane, *selected, dense_chain(binding, selected->capacity), target);
+  size_t index = 0;
+  while (selected->plans[index].rows < rows) {
+    ++index;
+  }
+  return run_chain(lane, selected->graphs[index], dense_chain(binding, selected->layout, selected->plans[index]), target);
 }
 
 
@@ -2409,7 +2519,8 @@ int xp_moe_template_capture(xp_lane_t lane, const xp_moe_layer_desc *desc, int64
   t->intermediate = signature.intermediate;
   t->capacity = capacity;
   t->moe = signature;
-  if (const int status = instantiate_template(*t, chain); status != XP_OK) {
+  t->graphs.resize(1);
+  if (const int status = instantiate_graph(t->graphs.front(), chain); status != XP_OK) {
     return status;
   }
   insert_template(lane, std::move(t));

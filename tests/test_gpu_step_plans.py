@@ -1,0 +1,108 @@
+"""Dense steps between a template's capacities: the plan each row count takes.
+
+A template of more than 64 rows keeps tile choices for several row counts; replays at a
+tile's edges must agree with fp64 whatever the choice (192 x 256 and 128 x 256 tiles, K splits
+that are no power of two, column splits, rotated weight streams, weight tile counts that do
+not divide over the XCDs), repeat bit for bit, and give the same bits through graph dispatch.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from crosspool_amd import _native
+from crosspool_amd.agent import FfnAgent
+from crosspool_amd.weights import DenseFfnWeights
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer(device, hidden, intermediate, dtype):
+    generator = torch.Generator(device=device).manual_seed(hidden + intermediate)
+    gate_up = (torch.randn((2 * intermediate, hidden), device=device, generator=generator) * 0.02).to(dtype)
+    down = (torch.randn((hidden, intermediate), device=device, generator=generator) * 0.02).to(dtype)
+    norm = (1 + 0.1 * torch.randn((hidden,), device=device, generator=generator)).to(dtype)
+    return gate_up, down, norm
+
+
+def _expected(rows, gate_up, down, norm):
+    """The step in fp64 with the path's rounding points."""
+
+    dtype = rows.dtype
+    x = rows.double()
+    x = (x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6) * norm.double()).to(dtype).double()
+    projected = (x @ gate_up.double().t()).to(dtype).double()
+    gate, up = projected[:, 0::2], projected[:, 1::2]
+    return (gate * torch.sigmoid(gate) * up).to(dtype).double() @ down.double().t()
+
+
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))
+@pytest.mark.parametrize(
+    "hidden,intermediate,capacity,rows_list",
+    (
+        (2560, 9728, 1024, (257, 517, 576, 577)),     # 192 x 256 gate_up, K splits of down
+        (1536, 8960, 512, (192, 193, 320, 321)),      # 70 weight tiles of 256
+        (5120, 3200, 2048, (1025, 1152, 2048)),       # 25 weight tiles, column splits
+        (4096, 1032, 128, (33, 64, 65, 128)),         # rotated weight streams, ragged N
+        (8192, 264, 64, (33, 64)),                    # the same at another multiple of 8 KB
+        (1032, 1000, 300, (65, 128, 129, 300)),       # ragged K and N, a capacity between two steps
+        (2048, 6144, 1024, (600, 640, 641)),          # 128 x 256 gate_up
+    ),
+)
+def test_steps_between_capacities(device, hidden, intermediate, capacity, rows_list, dtype):
+    gate_up, down, norm = _layer(device, hidden, intermediate, dtype)
+    generator = torch.Generator(device=device).manual_seed(5)
+    pool = torch.randn((capacity + 40, hidden), device=device, generator=generator).to(dtype)
+    slots = torch.randperm(pool.shape[0], device=device, generator=generator).to(torch.int32)
+    outputs = {}
+    for graph_dispatch in (False, True):
+        with FfnAgent(device, graph_dispatch=graph_dispatch) as agent:
+            agent.register_layer(instance_index=0, layer_ordinal=0, norm_weight=norm, eps=1e-6,
+                                 weights=DenseFfnWeights.from_tensors(gate_up, down))
+            agent.materialize(maximum_row_capacity=capacity)
+            for rows in rows_list + rows_list[:1]:
+                print(f"step plan {hidden}x{intermediate} {rows}/{capacity} {dtype} graph={graph_dispatch}", flush=True)
+                out = torch.zeros_like(pool)
+                agent.execute(instance_index=0, layer_ordinal=0, pool=pool, slots=slots, rows=rows, out_pool=out)
+                agent.check_health()
+                previous = outputs.setdefault(rows, out)
+                assert torch.equal(out.view(torch.int16), previous.view(torch.int16)), "replays differ"
+    for rows, out in outputs.items():
+        live = slots[:rows].long()
+        expected = _expected(pool[live], gate_up, down, norm)
+        # Sums in another order round a few values the other way: one ulp of activations and outputs.
+        error = (out[live].double() - expected).norm() / expected.norm()
+        ulp = 2.0**-8 if dtype is torch.bfloat16 else 2.0**-11
+        assert error <= ulp, f"{rows} rows: relative error {error:.2e}"
+        untouched = torch.ones(pool.shape[0], dtype=torch.bool, device=device)
+        untouched[live] = False
+        assert not out[untouched].any()
+
+
+def test_eager_step_runs_in_the_smallest_accepted_workspace(device):
+    # The eager step keeps the capacity's own choice where a workspace has no room for the
+    # refined one's K ranges, and refuses only what neither fits.
+    hidden, intermediate, rows = 2560, 9728, 640
+    gate_up, down, norm = _layer(device, hidden, intermediate, torch.bfloat16)
+    pool = torch.randn((700, hidden), device=device).bfloat16()
+    slots = torch.randperm(700, device=device)[:rows].to(torch.int32)
+    base = rows * (hidden + intermediate) * 2
+    scratch = _native.gemm_workspace_bytes(rows, hidden, intermediate, False) + _native.gemm_workspace_bytes(
+        rows, 2 * intermediate, hidden, True)
+    expected = _expected(pool[slots.long()], gate_up, down, norm)
+    import ctypes
+
+    def pointer(tensor):
+        return ctypes.c_void_p(tensor.data_ptr())
+
+    for nbytes in (_native.dense_workspace_bytes(rows, hidden, intermediate), (base + 255) // 256 * 256 + scratch):
+        print(f"eager step workspace {nbytes}", flush=True)
+        workspace = torch.empty(nbytes, dtype=torch.uint8, device=device)
+        out = torch.zeros_like(pool)
+        _native.call("xp_dense_step", pointer(pool), pointer(out), 700, pointer(slots), rows, hidden, intermediate,
+                     pointer(gate_up), pointer(down), pointer(norm), 1e-6, pointer(workspace), nbytes, None,
+                     ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        error = (out[slots.long()].double() - expected).norm() / expected.norm()
+        assert error <= 2.0**-8
