@@ -447,9 +447,10 @@ GemmChoice choose_step_tile(const GemmChoice &base, int64_t rows, int64_t n, int
     // A first launch of nearly whole rounds, and the remaining columns in a second one.
     const TileShape &shape = kTileShapes[tile.variant];
     const int64_t token_tiles = (rows + shape.bm - 1) / shape.bm;
-    for (int64_t weight_tiles = 1; weight_tiles * shape.bn < n; ++weight_tiles) {
-      const int64_t partial = token_tiles * weight_tiles % kComputeUnits;
-      if (token_tiles * weight_tiles < kComputeUnits * 3 / 4 || (partial != 0 && partial < kComputeUnits * 11 / 12)) {
+    for (int64_t rounds = 1; kComputeUnits * rounds / token_tiles * shape.bn < n; ++rounds) {
+      const int64_t weight_tiles = kComputeUnits * rounds / token_tiles;
+      const int64_t idle = kComputeUnits * rounds - token_tiles * weight_tiles;
+      if (weight_tiles == 0 || idle * 12 > kComputeUnits) {
         continue;
       }
       GemmChoice choice{GemmKind::Tile, tile.variant, k, 1};
@@ -772,22 +773,15 @@ KernelLaunch make_grouped_gemm(const GemmArgs &args, bool gated, int max_tiles, 
 // Routes per expert tile of the grouped split kernel: one 16-column MFMA token block.
 int grouped_split_rows() { return 16; }
 
-// K ranges per weight block: the most (1, 2, 4 or 8) that keep the expected live tiles'
-// workgroups within one round of one per CU, with every range at least two 128-wide chunks
-// long.  A workgroup at decode sizes is latency-bound (the tile table, the route slots,
-// then the weights and tokens, each a memory round trip), so a second round of
-// workgroups costs nearly as much as the first (Qwen3-30B-A3B gate_up at 1 token: 384
-// workgroups in two rounds 17.8 us).
-KernelLaunch make_grouped_split(const GemmArgs &args, bool gated, int max_tiles, int64_t live_tiles) {
+// K ranges per weight block: two (both waves of a workgroup on one block) where each still has
+// at least four 128-wide chunks.  Every pairing of 1 to 8 ranges with 1 to 8 waves, forced on the
+// Qwen3-30B-A3B layer and a 1024 x 512, 64-expert one at 1 to 64 tokens: this is the fastest or
+// within 2 % of it (gate_up K = 2048 at 32 tokens 185.7 us, one range 190.2; down K = 768 185.7,
+// two ranges 193.1).
+KernelLaunch make_grouped_split(const GemmArgs &args, bool gated, int max_tiles) {
   const int64_t row_blocks = (args.n + 15) / 16;
   const int64_t chunks = (args.k + 127) / 128;
-  auto nonempty = [&](int64_t ranges) { return (ranges - 1) * ((chunks + ranges - 1) / ranges) < chunks; };
-  auto workgroups = [&](int64_t ranges) { return (row_blocks * ranges + kSplitWaves - 1) / kSplitWaves * live_tiles; };
-  int64_t ksplit = 1;
-  while (ksplit < kSplitWaves && 4 * ksplit <= chunks && nonempty(2 * ksplit) &&
-         workgroups(2 * ksplit) <= kComputeUnits) {
-    ksplit *= 2;
-  }
+  const int64_t ksplit = chunks >= 4 * kGroupedSplitWaves ? kGroupedSplitWaves : 1;
   GemmArgs record = args;
   record.k_split = ksplit;
   record.k_slice = (chunks + ksplit - 1) / ksplit * 128;
@@ -795,9 +789,9 @@ KernelLaunch make_grouped_split(const GemmArgs &args, bool gated, int max_tiles,
   KernelLaunch kernel;
   kernel.func = args.payload == kPayloadF16 ? GroupedKernels<F16Payload>::split(gated)
                                             : GroupedKernels<Bf16Payload>::split(gated);
-  kernel.grid = dim3(static_cast<unsigned>((row_blocks * ksplit + kSplitWaves - 1) / kSplitWaves),
+  kernel.grid = dim3(static_cast<unsigned>((row_blocks * ksplit + kGroupedSplitWaves - 1) / kGroupedSplitWaves),
                      static_cast<unsigned>(max_tiles), 1);
-  kernel.block = dim3(64 * kSplitWaves, 1, 1);
+  kernel.block = dim3(64 * kGroupedSplitWaves, 1, 1);
   kernel.set_args(record);
   return kernel;
 }

@@ -53,11 +53,8 @@ constexpr int kNarrowDecodeTile = 4;  // 64 x 64
 // Chunks in flight per wave of the grouped split kernel.  Its workgroups are short (a wave
 // streams one 16-row block of one expert: 24 KB of Qwen3-30B-A3B's down projection), so
 // the fixed cost of each (the tile table, the route slots, the first round trip) weighs
-// more than the depth of its ring: at depth 2 the kernel takes 107 VGPRs and two
-// workgroups share a CU, one streaming while the other starts or ends.  Qwen3-30B-A3B
-// layer at 8 / 32 / 64 tokens: 121.5 / 215.7 / 238.1 us at depth 4 (160 VGPRs, one
-// workgroup per CU), 115.0 / 201.2 / 223.3 at depth 2; depth 3 (128 VGPRs, two per CU, and
-// chunk counts that do not divide into its groups) 122.4 / 217.0 / 238.7.
+// more than the depth of its ring: at depth 2 the kernel takes at most 128 VGPRs and a SIMD
+// holds four of its waves (depth 4, with half as many: 6 % slower at 8 and 32 tokens).
 constexpr int kGroupedSplitDepth = 2;
 
 // How a tile launch loads its weights, each its own instantiation (a per-load branch on an

@@ -788,14 +788,12 @@ int make_experts_launches(const ExpertsBinding &b, int64_t capacity, ExpertsLaun
       return fail(XP_ERROR_STATE, "no grouped tile kernel for this expert tile table");
     }
   } else {
-    // Few routes per expert: each touched expert's weights streamed by the grouped split
-    // kernel; about one tile per touched expert.
+    // Few routes per expert: each touched expert's weights streamed by the grouped split kernel.
     if (moe_tile_rows(MoeTile::Small) != grouped_split_rows()) {
       return fail(XP_ERROR_STATE, "expert tile table and grouped split kernel disagree on the tile rows");
     }
-    const int64_t live_tiles = b.experts < capacity_routes ? b.experts : capacity_routes;
-    out.gate_up = make_grouped_split(up, true, max_tiles, live_tiles);
-    out.down = make_grouped_split(dn, false, max_tiles, live_tiles);
+    out.gate_up = make_grouped_split(up, true, max_tiles);
+    out.down = make_grouped_split(dn, false, max_tiles);
   }
 
   MoeCombineArgs combine{};
@@ -1844,10 +1842,11 @@ int xp_template_capture(xp_lane_t lane, int64_t hidden, int64_t intermediate, in
     return status;
   }
   XP_REQUIRE(capacity > 0, "template capacity must be positive");
-  const size_t needed = dense_workspace(capacity, hidden, intermediate).bytes;
-  if (needed > lane->workspace_bytes) {
-    return fail(XP_ERROR_CAPACITY, "Lane workspace is smaller than the template needs (" + std::to_string(needed) +
-                                       " bytes)");
+  std::vector<DensePlan> plans = plan_dense_template(capacity, hidden, intermediate);
+  const DenseWorkspace layout = dense_workspace(capacity, hidden, intermediate, plans.data(), plans.size());
+  if (layout.bytes > lane->workspace_bytes) {
+    return fail(XP_ERROR_CAPACITY, "Lane workspace is smaller than the template needs (" +
+                                       std::to_string(layout.bytes) + " bytes)");
   }
   std::lock_guard<std::mutex> guard(lane->mutex);
   for (const auto &t : lane->templates) {
@@ -1871,8 +1870,8 @@ int xp_template_capture(xp_lane_t lane, int64_t hidden, int64_t intermediate, in
   t->intermediate = intermediate;
   t->payload = payload;
   t->capacity = capacity;
-  t->plans = plan_dense_template(capacity, hidden, intermediate);
-  t->layout = dense_workspace(capacity, hidden, intermediate, t->plans.data(), t->plans.size());
+  t->plans = std::move(plans);
+  t->layout = layout;
   t->graphs.resize(t->plans.size());
   if (const int status = instantiate_graph(t->graphs.back(), dense_chain(binding, t->layout, t->plans.back()));
       status != XP_OK) {

@@ -448,9 +448,8 @@ GemmLaunch make_gemm(const GemmArgs &args, int64_t capacity, bool gated, GemmCho
 KernelLaunch make_grouped_gemm(const GemmArgs &args, bool gated, int max_tiles, MoeTile tile);
 int grouped_tile_rows(MoeTile tile);
 // The grouped projection for few routes per expert, on the grouped split kernel: tiles of
-// grouped_split_rows() sorted positions, `live_tiles` the expected number of table entries
-// in use (it sizes the K split).
-KernelLaunch make_grouped_split(const GemmArgs &args, bool gated, int max_tiles, int64_t live_tiles);
+// grouped_split_rows() sorted positions.
+KernelLaunch make_grouped_split(const GemmArgs &args, bool gated, int max_tiles);
 int grouped_split_rows();
 std::string gemm_name(GemmChoice choice, bool gated);
 
