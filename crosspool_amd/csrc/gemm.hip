@@ -627,12 +627,14 @@ GemmLaunch make_gemm(const GemmArgs &args, int64_t capacity, bool gated, GemmCho
   if (choice.kind == GemmKind::Split) {
     // choose_split is only consulted up to kSplitMaxRows rows (and the fused gather up to
     // one token group).
-    const int64_t row_blocks = (args.n + 15) / 16;
     const int64_t per_group = kSplitWaves / choice.k_split;
+    // 8-row weight blocks while 16-row ones would fill at most half the CUs.
+    const bool half = ((args.n + 15) / 16 + per_group - 1) / per_group * 2 <= kComputeUnits;
+    const int64_t row_blocks = half ? (args.n + 7) / 8 : (args.n + 15) / 16;
     // The gather fuses into one token group (gate_up of a Dense step, the MoE router).
     const bool gather = fused_gather && choice.variant == 1;
-    kernel.func = f16 ? DenseKernels<F16Payload>::split(gated, choice.variant, gather)
-                      : DenseKernels<Bf16Payload>::split(gated, choice.variant, gather);
+    kernel.func = f16 ? DenseKernels<F16Payload>::split(gated, choice.variant, gather, half)
+                      : DenseKernels<Bf16Payload>::split(gated, choice.variant, gather, half);
     kernel.grid = dim3(static_cast<unsigned>((row_blocks + per_group - 1) / per_group), 1, 1);
     kernel.block = dim3(64 * kSplitWaves, 1, 1);
     // Dynamic LDS beyond 64 KB: launch() opts the function in (enable_large_lds).

@@ -10,18 +10,23 @@ const void *kernel_address(Kernel kernel) {
   return reinterpret_cast<const void *>(kernel);
 }
 
-template <class P>
-const void *DenseKernels<P>::split(bool gated, int groups, bool gather) {
+template <class P, int HALVES>
+const void *split_kernel(bool gated, int groups, bool gather) {
   if (gather) {
-    return gated ? kernel_address(&split_gemm_kernel<split_depth(1), 1, true, true, P>)
-                 : kernel_address(&split_gemm_kernel<split_depth(1), 1, false, true, P>);
+    return gated ? kernel_address(&split_gemm_kernel<split_depth(1), 1, true, true, P, HALVES>)
+                 : kernel_address(&split_gemm_kernel<split_depth(1), 1, false, true, P, HALVES>);
   }
   if (groups == 1) {
-    return gated ? kernel_address(&split_gemm_kernel<split_depth(1), 1, true, false, P>)
-                 : kernel_address(&split_gemm_kernel<split_depth(1), 1, false, false, P>);
+    return gated ? kernel_address(&split_gemm_kernel<split_depth(1), 1, true, false, P, HALVES>)
+                 : kernel_address(&split_gemm_kernel<split_depth(1), 1, false, false, P, HALVES>);
   }
-  return gated ? kernel_address(&split_gemm_kernel<split_depth(2), 2, true, false, P>)
-               : kernel_address(&split_gemm_kernel<split_depth(2), 2, false, false, P>);
+  return gated ? kernel_address(&split_gemm_kernel<split_depth(2), 2, true, false, P, HALVES>)
+               : kernel_address(&split_gemm_kernel<split_depth(2), 2, false, false, P, HALVES>);
+}
+
+template <class P>
+const void *DenseKernels<P>::split(bool gated, int groups, bool gather, bool half) {
+  return half ? split_kernel<P, 1>(gated, groups, gather) : split_kernel<P, 2>(gated, groups, gather);
 }
 
 template <class P>

@@ -259,8 +259,14 @@ constexpr int kSplitMaxGroups = 2;
 // are in flight; the token pieces are then read from LDS instead of L2.  Dynamic LDS:
 // min(capacity, 8) x (K + 16) bf16 (the 32-byte row padding puts the 16 pieces of one read
 // in distinct bank slots).
-template <int DEPTH, int TG, bool GATED, bool GATHER = false, class P = Bf16Payload>
+//
+// HALVES: 8-row halves of a weight block per wave.  One instead of two doubles the workgroups of
+// a projection whose 16-row blocks leave half the CUs idle; the K ranges and their order are the
+// same, and so are the bits.  Captured 28-layer Qwen3-0.6B stack at 7 rows (96 and 64 workgroups
+// before) 518 -> 469 us; Qwen3-1.7B layer at 1 / 4 rows (down: 128) 24.4 / 25.2 -> 21.6 / 22.2.
+template <int DEPTH, int TG, bool GATED, bool GATHER = false, class P = Bf16Payload, int HALVES = 2>
 __global__ __launch_bounds__(64 * kSplitWaves) void split_gemm_kernel(GemmArgs a) {
+  constexpr int ROWS = 8 * HALVES;  // weight rows of a block
   static_assert(!GATHER || TG == 1, "the fused gather stages one token group");
   extern __shared__ __attribute__((aligned(16))) uint16_t staged[];
   const int lane = threadIdx.x & 63;
@@ -272,19 +278,21 @@ __global__ __launch_bounds__(64 * kSplitWaves) void split_gemm_kernel(GemmArgs a
   const int ksplit = static_cast<int>(a.k_split);
   const int part = wave % ksplit;
   const int64_t rb = static_cast<int64_t>(blockIdx.x) * (kSplitWaves / ksplit) + wave / ksplit;
-  const int64_t row_blocks = (a.n + 15) / 16;
+  const int64_t row_blocks = (a.n + ROWS - 1) / ROWS;
   const bool active = rb < row_blocks;
   const u32x4 zero = {0u, 0u, 0u, 0u};
   const int64_t rs = a.k + 16;  // staged row stride in elements (GATHER)
   // GATHER: rows staged in LDS, the capacity's: rows past them are zero.
   const int staged_rows = a.capacity < kSplitGroupTokens ? static_cast<int>(a.capacity) : kSplitGroupTokens;
 
-  // acc[g][h]: token group g, weight rows 16 rb + 8 h + [0, 8).
-  f32x4 acc[TG][2];
+  // acc[g][h]: token group g, weight rows ROWS rb + 8 h + [0, 8).
+  f32x4 acc[TG][HALVES];
 #pragma unroll
   for (int g = 0; g < TG; ++g) {
-    acc[g][0] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    acc[g][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h) {
+      acc[g][h] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
   }
 
   const int k0 = part * static_cast<int>(a.k_slice);
@@ -299,10 +307,10 @@ __global__ __launch_bounds__(64 * kSplitWaves) void split_gemm_kernel(GemmArgs a
   const int lane_valid = static_cast<int>(a.k) - k0 - piece * 8;
   // Row blocks start at different chunks of their range (stride-7 rotation), spreading the
   // concurrently streamed addresses over the memory channels.
-  const int rotation = static_cast<int>((rb * 7) % chunks);
+  const int rotation = static_cast<int>((rb * ROWS / 16 * 7) % chunks);
   const __amdgpu_buffer_rsrc_t w_rsrc = make_rsrc(a.w, static_cast<uint32_t>(a.n * a.k * 2));
   const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(a.x, static_cast<uint32_t>(a.rows * a.ldx * 2));
-  const uint32_t w_off = static_cast<uint32_t>(((rb * 16 + row) * a.k + k0 + piece * 8) * 2);
+  const uint32_t w_off = static_cast<uint32_t>(((rb * ROWS + row) * a.k + k0 + piece * 8) * 2);
   const uint32_t w_half = static_cast<uint32_t>(8 * a.k * 2);  // rows 8 .. 15 of the block
   const uint32_t x_off = static_cast<uint32_t>((row * a.ldx + k0 + piece * 8) * 2);
   const uint32_t x_group = static_cast<uint32_t>(kSplitGroupTokens * a.ldx * 2);
@@ -311,19 +319,19 @@ __global__ __launch_bounds__(64 * kSplitWaves) void split_gemm_kernel(GemmArgs a
     return (c < chunks ? c : c - chunks) * 128;
   };
 
-  // Per chunk: w[2 line + h] = line `line` (K columns 64 line .. 64 line + 63 of the chunk)
+  // Per chunk: w[HALVES line + h] = line `line` (K columns 64 line .. 64 line + 63 of the chunk)
   // of rows 8 h + [0, 8); x[line][g] the matching pieces of token group g.
   constexpr int XG = GATHER ? 0 : TG;
-  u32x4 wbuf[DEPTH][4];
+  u32x4 wbuf[DEPTH][2 * HALVES];
   u32x4 xbuf[DEPTH][2][XG > 0 ? XG : 1];
-  auto load_chunk = [&](int chunk, u32x4 (&w)[4], u32x4 (&x)[2][XG > 0 ? XG : 1]) {
+  auto load_chunk = [&](int chunk, u32x4 (&w)[2 * HALVES], u32x4 (&x)[2][XG > 0 ? XG : 1]) {
     const bool in_range = chunk < chunks;
     const uint32_t column = static_cast<uint32_t>(column_of(chunk)) * 2;
 #pragma unroll
     for (int line = 0; line < 2; ++line) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        w[2 * line + h] = buffer_load16<kLoadNontemporal>(
+      for (int h = 0; h < HALVES; ++h) {
+        w[HALVES * line + h] = buffer_load16<kLoadNontemporal>(
             w_rsrc, in_range ? w_off + h * w_half + column + line * 128 : kOutOfRange);
       }
 #pragma unroll
@@ -332,13 +340,16 @@ __global__ __launch_bounds__(64 * kSplitWaves) void split_gemm_kernel(GemmArgs a
       }
     }
   };
-  auto compute_chunk = [&](int chunk, const u32x4 (&w)[4], const u32x4 (&x)[2][XG > 0 ? XG : 1]) {
+  auto compute_chunk = [&](int chunk, const u32x4 (&w)[2 * HALVES], const u32x4 (&x)[2][XG > 0 ? XG : 1]) {
     const int column = chunk < chunks ? column_of(chunk) : 0;
 #pragma unroll
     for (int line = 0; line < 2; ++line) {
       const bool valid = column + line * 64 < lane_valid;
-      const u32x4 w0 = valid ? w[2 * line] : zero;
-      const u32x4 w1 = valid ? w[2 * line + 1] : zero;
+      u32x4 wk[HALVES];
+#pragma unroll
+      for (int h = 0; h < HALVES; ++h) {
+        wk[h] = valid ? w[HALVES * line + h] : zero;
+      }
 #pragma unroll
       for (int g = 0; g < TG; ++g) {
         u32x4 xk;
@@ -347,8 +358,10 @@ __global__ __launch_bounds__(64 * kSplitWaves) void split_gemm_kernel(GemmArgs a
         } else {
           xk = valid ? x[line][g] : zero;
         }
-        acc[g][0] = P::mfma16(w0, xk, acc[g][0]);
-        acc[g][1] = P::mfma16(w1, xk, acc[g][1]);
+#pragma unroll
+        for (int h = 0; h < HALVES; ++h) {
+          acc[g][h] = P::mfma16(wk[h], xk, acc[g][h]);
+        }
       }
     }
   };
@@ -396,12 +409,14 @@ __global__ __launch_bounds__(64 * kSplitWaves) void split_gemm_kernel(GemmArgs a
 
   // Fixed-order sum of the K ranges of each row block: range 0's wave adds ranges
   // 1 .. KSPLIT-1 in order.
-  __shared__ f32x4 partial[kSplitWaves][TG][2][64];
+  __shared__ f32x4 partial[kSplitWaves][TG][HALVES][64];
   if (ksplit > 1) {
 #pragma unroll
     for (int g = 0; g < TG; ++g) {
-      partial[wave][g][0][lane] = acc[g][0];
-      partial[wave][g][1][lane] = acc[g][1];
+#pragma unroll
+      for (int h = 0; h < HALVES; ++h) {
+        partial[wave][g][h][lane] = acc[g][h];
+      }
     }
     __syncthreads();
     if (part != 0) {
@@ -410,7 +425,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void split_gemm_kernel(GemmArgs a
 #pragma unroll
     for (int g = 0; g < TG; ++g) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
+      for (int h = 0; h < HALVES; ++h) {
         for (int p = 1; p < ksplit; ++p) {
           acc[g][h] += partial[wave + p][g][h][lane];
         }
@@ -423,12 +438,12 @@ __global__ __launch_bounds__(64 * kSplitWaves) void split_gemm_kernel(GemmArgs a
 
   // Lane (i, q) holds D[4 q + v][i], v = 0 .. 3.  The lanes with q < 2 and i < 8 add the odd
   // pieces' block from lane + 40 (D[4 q + 8 + v][i + 8]) and then hold weight rows
-  // 16 rb + 8 h + 4 q + v for token 8 g + i.
-  f32x4 sum[TG][2];
+  // ROWS rb + 8 h + 4 q + v for token 8 g + i.
+  f32x4 sum[TG][HALVES];
 #pragma unroll
   for (int g = 0; g < TG; ++g) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < HALVES; ++h) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         sum[g][h][v] = acc[g][h][v] + __shfl(acc[g][h][v], lane + 40, kWave);
@@ -449,8 +464,8 @@ __global__ __launch_bounds__(64 * kSplitWaves) void split_gemm_kernel(GemmArgs a
       continue;
     }
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int64_t n = rb * 16 + 8 * h + 4 * kq;
+    for (int h = 0; h < HALVES; ++h) {
+      const int64_t n = rb * ROWS + 8 * h + 4 * kq;
       if (n >= a.n) {
         continue;
       }

@@ -72,7 +72,8 @@ struct DenseKernels {
   // (Four groups, 32 tokens, were measured and dropped: the token pieces read from L2 for each
   // weight line then cost more than the tile kernels, 60-77 us against 41-43 us for Qwen3-8B
   // gate_up at 17-32 rows.)
-  static const void *split(bool gated, int groups, bool gather);
+  // `half`: on 8-row weight blocks.
+  static const void *split(bool gated, int groups, bool gather, bool half);
   // The persistent split kernel with the gather fused (one token group).
   static const void *split_gathered(bool gated);
   static const void *stream(bool gated, bool gather);

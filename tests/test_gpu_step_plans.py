@@ -80,6 +80,29 @@ def test_steps_between_capacities(device, hidden, intermediate, capacity, rows_l
         assert not out[untouched].any()
 
 
+# 8-row weight blocks (16-row ones would fill at most half the CUs): N around the last block,
+# K ranges that end inside a chunk, one and two token groups, gate_up with the gather fused.
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))
+@pytest.mark.parametrize("hidden,intermediate", ((1024, 3072), (1016, 1000), (264, 40), (2048, 6144)))
+def test_half_block_steps(device, hidden, intermediate, dtype):
+    gate_up, down, norm = _layer(device, hidden, intermediate, dtype)
+    pool = torch.randn((64, hidden), device=device, generator=torch.Generator(device=device).manual_seed(9)).to(dtype)
+    slots = torch.randperm(64, device=device).to(torch.int32)
+    with FfnAgent(device) as agent:
+        agent.register_layer(instance_index=0, layer_ordinal=0, norm_weight=norm, eps=1e-6,
+                             weights=DenseFfnWeights.from_tensors(gate_up, down))
+        agent.materialize(maximum_row_capacity=16)
+        for rows in (1, 2, 7, 8, 9, 16):
+            print(f"half blocks {hidden}x{intermediate} {rows} {dtype}", flush=True)
+            out = torch.zeros_like(pool)
+            agent.execute(instance_index=0, layer_ordinal=0, pool=pool, slots=slots, rows=rows, out_pool=out)
+            agent.check_health()
+            live = slots[:rows].long()
+            expected = _expected(pool[live], gate_up, down, norm)
+            error = (out[live].double() - expected).norm() / expected.norm()
+            assert error <= (2.0**-8 if dtype is torch.bfloat16 else 2.0**-11), f"{rows} rows: {error:.2e}"
+
+
 def test_eager_step_runs_in_the_smallest_accepted_workspace(device):
     # The eager step keeps the capacity's own choice where a workspace has no room for the
     # refined one's K ranges, and refuses only what neither fits.
