@@ -1619,13 +1619,14 @@ __device__ __forceinline__ void static_for(F &&f) {
 // 470 -> 461 us, of a hidden-1536 layer (70) at 896 rows on 128 x 256 tiles 67.6 -> 55.8,
 // Qwen3-4B down (10) at 4096 rows 207 -> 194; worst Qwen3-4B gate_up (76) at 2048 rows, 184 ->
 // 188.  With more than 8 token tiles and even weight tiles the grid coordinates are used as
-// they are (blocks took 3 % longer; runs 2 % less on 256 x 256 tiles, 5 % more on 256 x 128).
+// they are (blocks took 3 % longer; runs 2 % less on 256 x 256 tiles, 5 % more on 256 x 128), and
+// so are those of a single row or column of tiles, where there is nothing to share.
 // The results are wave-uniform; readfirstlane keeps them (and the buffer resources built from
 // them) in scalar registers.
 __device__ __forceinline__ void tile_coordinates(int &tn, int &tm) {
   const int nx = static_cast<int>(gridDim.x);
   const int ny = static_cast<int>(gridDim.y);
-  if (nx % 8 == 0 && ny > 8) {
+  if (nx == 1 || ny == 1 || (nx % 8 == 0 && ny > 8)) {
     tn = static_cast<int>(blockIdx.x);
     tm = static_cast<int>(blockIdx.y);
     return;

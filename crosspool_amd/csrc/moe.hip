@@ -501,35 +501,36 @@ unsigned blocks_for(int64_t items, int64_t per_block) {
 
 int moe_tile_rows(MoeTile tile) { return tile == MoeTile::Small ? grouped_split_rows() : grouped_tile_rows(tile); }
 
-// Few routes per expert (at most 4 on average) stream each expert's weights through the
-// grouped split kernel in 16-route tiles; more take the grouped tile kernel on the shortest
-// expert tile that holds most experts' routes.  An expert's weights are read once per tile
-// of its routes, and the LDS a tile's token rows do not take holds weight slabs in flight
-// (the grouped projections are bound by the weight bytes each CU has in flight), so:
-// 64-row tiles (two workgroups per CU, each with two of its three 64 x 128 weight slabs in
-// flight) up to 40 routes per expert on
-// average, 128-row tiles with the weights loaded nontemporally up to 80, 128-row tiles with
-// plain loads (an expert split over two tiles finds its weights in the last-level cache
-// for the second) up to 160, 256-row tiles above.  Measured at the Qwen3-30B-A3B shape
-// (128 experts, top-8), layer us against the 256-row tile everywhere: 256 tokens 335 -> 288,
-// 512 357 -> 304, 1024 391 -> 332, 2048 431 -> 418, 4096 unchanged (647 against 652 on
-// 128-row tiles); 128 tokens (8 routes per expert) 298 us on 16-route tiles -> 279 on 64-row
-// tiles, while at 48 / 64 tokens (3 / 4 routes per expert) the 64-row tiles lost (254 / 263
-// -> 263 / 270 us).  (Those 64-row figures are of a 64 x 256 tile, one workgroup per CU; the
-// 64 x 128 tile at two per CU since took 256 / 512 tokens to 255 / 265 us, while in the
-// 80-route regime it won below the capacity's 1024 tokens and lost at them: 377 against
-// 319 us, so the thresholds stand.)
-MoeTile choose_moe_tile(int64_t routes, int64_t experts) {
+// Few routes per expert stream each expert's weights through the grouped split kernel in
+// 16-route tiles; more take the grouped tile kernel on the shortest expert tile that holds most
+// experts' routes.  An expert's weights are read once per tile of its routes, and the LDS a
+// tile's token rows do not take holds weight slabs in flight (the grouped projections are bound
+// by the weight bytes each CU has in flight).  The thresholds are about where neighbours cross,
+// by routes per expert on average (layer us at the Qwen3-30B-A3B shape, 128 experts, top-8, then
+// of a 1024 x 512, 64-expert top-6 layer): 16-route tiles against 64-row ones (two workgroups per
+// CU) at 3 / 4 / 8 routes 207 / 218 / 256 and 233 / 238 / 245, at 3.8 / 6 routes 63.0 / 65.8
+// and 60.0 / 61.3; those against 128-row ones with nontemporal weight loads at 40 / 48 / 56
+// routes 268 / 289 / 318 and 300 / 307 / 312, at 36 / 60 routes 65.9 / 88.8 and 69.6 / 73.7;
+// those against 128-row ones with plain loads (an expert split over two tiles finds its weights
+// in the last-level cache for the second) at 96 / 112 / 128 routes 355 / 380 / 457 and 366 / 379
+// / 396; and those against 256-row ones at 128 / 144 / 160 routes 396 / 443 / 485 and 424 / 431
+// / 463.  Experts of less than kRereadExpertBytes of gate_up weights gain nothing from the
+// second reading: 108 / 120 / 144 routes 114.1 / 111.6 / 118.7 on 128-row tiles against 102.0 /
+// 107.5 / 114.4 on 256-row ones.  192-row tiles were the fastest only there (106.9 / 112.2 at
+// 120 / 144; the large layer at 128 routes 431).
+constexpr int64_t kRereadExpertBytes = int64_t{4} << 20;
+
+MoeTile choose_moe_tile(int64_t routes, int64_t experts, int64_t gate_up_bytes) {
   if (routes <= 4 * experts) {
     return MoeTile::Small;
   }
-  if (routes <= 40 * experts) {
+  if (routes <= 52 * experts) {
     return MoeTile::Rows64;
   }
-  if (routes <= 80 * experts) {
+  if (routes <= 104 * experts) {
     return MoeTile::Rows128Stream;
   }
-  return routes <= 160 * experts ? MoeTile::Rows128 : MoeTile::Rows256;
+  return routes <= 136 * experts && gate_up_bytes >= kRereadExpertBytes ? MoeTile::Rows128 : MoeTile::Rows256;
 }
 
 template <class P>

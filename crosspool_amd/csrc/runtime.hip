@@ -96,14 +96,22 @@ int64_t plan_row_step(int64_t capacity) {
   return (capacity + unit - 1) / unit * kPlanRowStep;
 }
 
+std::vector<int64_t> template_plan_rows(int64_t capacity) {
+  std::vector<int64_t> plans;
+  const int64_t step = plan_row_step(capacity);
+  for (int64_t rows = step; rows < capacity; rows += step) {
+    plans.push_back(rows);
+  }
+  plans.push_back(capacity);
+  return plans;
+}
+
 std::vector<DensePlan> plan_dense_template(int64_t capacity, int64_t hidden, int64_t intermediate) {
   std::vector<DensePlan> plans;
   const DensePlan base = plan_dense_capacity(capacity, hidden, intermediate);
-  const int64_t step = plan_row_step(capacity);
-  for (int64_t rows = step; rows < capacity; rows += step) {
+  for (const int64_t rows : template_plan_rows(capacity)) {
     plans.push_back(refine_plan(base, rows, hidden, intermediate));
   }
-  plans.push_back(refine_plan(base, capacity, hidden, intermediate));
   return plans;
 }
 
@@ -391,10 +399,11 @@ struct Template {
   int32_t payload = kPayloadBf16;
   int64_t capacity = 0;
   xp_moe_layer_desc moe{};  // MoE templates: the signature they were captured for
-  std::vector<DensePlan> plans;  // Dense templates, by rows; the last serves the capacity
+  std::vector<int64_t> plan_rows;  // increasing; the last is the capacity
+  std::vector<DensePlan> plans;    // Dense templates: one per plan_rows
   DenseWorkspace layout{};
-  // One per plan (MoE templates: one).  The capacity's is instantiated at capture, the others
-  // at their first replay through graph dispatch.
+  // One per plan.  The capacity's is instantiated at capture, the others at their first
+  // replay through graph dispatch.
   std::vector<std::unique_ptr<TemplateGraph>> graphs;
 };
 
@@ -670,7 +679,7 @@ RouterLaunches make_router_launches(const RouterBinding &b, int64_t capacity) {
 }
 
 // Experts kernels (route sort, grouped gate_up, grouped down, combine) for `rows` live rows,
-// with the tile choice, the tile table bound and the grids of `capacity` rows.
+// with the tile choice, the tile table bound and the grids of the plan's rows.
 struct ExpertsBinding {
   const uint16_t *x;  // [rows, hidden] token rows
   const uint16_t *w_gate_up;
@@ -703,7 +712,9 @@ struct ExpertsLaunches {
   KernelLaunch combine;
 };
 
-int make_experts_launches(const ExpertsBinding &b, int64_t capacity, ExpertsLaunches &out) {
+// `plan_rows`: the rows (at most the capacity the workspace is laid out for) that the tile
+// choice, the tile table and the grids serve.
+int make_experts_launches(const ExpertsBinding &b, int64_t capacity, int64_t plan_rows, ExpertsLaunches &out) {
   const MoeWorkspace layout = moe_workspace(capacity, b.hidden, b.intermediate, b.experts, b.topk);
   int32_t *expert_end = reinterpret_cast<int32_t *>(b.workspace + layout.expert_end);
   int32_t *sorted_route = reinterpret_cast<int32_t *>(b.workspace + layout.sorted_route);
@@ -713,10 +724,10 @@ int make_experts_launches(const ExpertsBinding &b, int64_t capacity, ExpertsLaun
   uint16_t *activated = reinterpret_cast<uint16_t *>(b.workspace + layout.activated);
   uint16_t *route_out = reinterpret_cast<uint16_t *>(b.workspace + layout.route_out);
   const int64_t routes = b.rows * b.topk;
-  const int64_t capacity_routes = capacity * b.topk;
-  const MoeTile tile = choose_moe_tile(capacity_routes, b.experts);
+  const int64_t plan_routes = plan_rows * b.topk;
+  const MoeTile tile = choose_moe_tile(plan_routes, b.experts, 4 * b.intermediate * b.hidden);
   const int tile_rows = moe_tile_rows(tile);
-  const int max_tiles = moe_tile_bound(capacity_routes, b.experts, tile_rows);
+  const int max_tiles = moe_tile_bound(plan_routes, b.experts, tile_rows);
   XP_REQUIRE(max_tiles <= 65535, "too many expert tiles for one call");
 
   MoeSortArgs sort{};
@@ -802,7 +813,7 @@ int make_experts_launches(const ExpertsBinding &b, int64_t capacity, ExpertsLaun
   combine.out = b.out;
   combine.slots = b.out_slots;
   combine.out_rows = b.out_rows;
-  combine.rows = capacity;
+  combine.rows = plan_rows;
   combine.hidden = b.hidden;
   combine.topk = static_cast<int32_t>(b.topk);
   combine.experts = static_cast<int32_t>(b.experts);
@@ -901,8 +912,9 @@ int validate_moe_capacity(const xp_moe_layer_desc &d, int64_t capacity) {
 }
 
 // One MoE mailbox step: gather (+ RMSNorm) into the batch, Router, finalisation (shared
-// experts only), Experts with the combine scattered to the slots of pool_out.  Grids and
-// kernel choices follow `capacity`; the argument records carry the live rows.
+// experts only), Experts with the combine scattered to the slots of pool_out.  Grids and kernel
+// choices follow `capacity`, the Experts' the plan's rows (as a Dense template's plans); the
+// argument records carry the live rows.
 struct MoeStepBinding {
   const uint16_t *pool_in;
   uint16_t *pool_out;
@@ -913,7 +925,7 @@ struct MoeStepBinding {
   uint32_t *fault;
 };
 
-int make_moe_step(const Layer &layer, const MoeStepBinding &b, int64_t capacity, StepChain &chain) {
+int make_moe_step(const Layer &layer, const MoeStepBinding &b, int64_t capacity, int64_t plan_rows, StepChain &chain) {
   const xp_moe_layer_desc &d = layer.moe;
   const MoeStepWorkspace layout = moe_step_workspace(d, capacity);
   uint16_t *batch = reinterpret_cast<uint16_t *>(b.workspace + layout.batch);
@@ -925,7 +937,7 @@ int make_moe_step(const Layer &layer, const MoeStepBinding &b, int64_t capacity,
 
   // At decode sizes the gather runs inside the router projection and the TopK inside the
   // route sort (two launches fewer; the same kernels' code, so the same bits).  Both follow
-  // from the capacity, so a template's node list matches every replay's.
+  // from the capacity.
   const bool fuse_gather = router_gather_fusable(d, capacity);
   const bool fuse_topk = capacity <= kMoeFusedTopkRows && topk == d.routed_topk;
   int32_t payload = kPayloadBf16;
@@ -1028,7 +1040,7 @@ int make_moe_step(const Layer &layer, const MoeStepBinding &b, int64_t capacity,
     experts.fused_topk = &routing.topk_args;
   }
   ExpertsLaunches launches;
-  if (const int status = make_experts_launches(experts, capacity, launches); status != XP_OK) {
+  if (const int status = make_experts_launches(experts, capacity, plan_rows, launches); status != XP_OK) {
     return status;
   }
   chain.add(launches.sort);
@@ -1870,6 +1882,7 @@ int xp_template_capture(xp_lane_t lane, int64_t hidden, int64_t intermediate, in
   t->intermediate = intermediate;
   t->payload = payload;
   t->capacity = capacity;
+  t->plan_rows = template_plan_rows(capacity);
   t->plans = std::move(plans);
   t->layout = layout;
   t->graphs.resize(t->plans.size());
@@ -1943,6 +1956,8 @@ int xp_replay(xp_lane_t lane, int instance_index, int layer_ordinal, int64_t row
   }
   // NULL is the legacy default stream, as for every other entry point.
   const hipStream_t target = static_cast<hipStream_t>(stream);
+  const size_t index = static_cast<size_t>(
+      std::lower_bound(selected->plan_rows.begin(), selected->plan_rows.end(), rows) - selected->plan_rows.begin());
   if (layer.kind == XP_LAYER_MOE) {
     MoeStepBinding binding{};
     binding.pool_in = static_cast<const uint16_t *>(pool_in);
@@ -1953,10 +1968,11 @@ int xp_replay(xp_lane_t lane, int instance_index, int layer_ordinal, int64_t row
     binding.workspace = lane->workspace;
     binding.fault = lane->fault;
     StepChain chain;
-    if (const int status = make_moe_step(layer, binding, selected->capacity, chain); status != XP_OK) {
+    if (const int status = make_moe_step(layer, binding, selected->capacity, selected->plan_rows[index], chain);
+        status != XP_OK) {
       return status;
     }
-    return run_chain(lane, selected->graphs.front(), chain, target);
+    return run_chain(lane, selected->graphs[index], chain, target);
   }
   DenseBinding binding{};
   binding.pool_in = static_cast<const uint16_t *>(pool_in);
@@ -1973,10 +1989,6 @@ int xp_replay(xp_lane_t lane, int instance_index, int layer_ordinal, int64_t row
   binding.workspace = lane->workspace;
   binding.fault = lane->fault;
   binding.payload = layer.payload;
-  size_t index = 0;
-  while (selected->plans[index].rows < rows) {
-    ++index;
-  }
   return run_chain(lane, selected->graphs[index], dense_chain(binding, selected->layout, selected->plans[index]), target);
 }
 
@@ -2391,7 +2403,7 @@ int xp_moe_experts(const void *hidden_states, int64_t rows, int64_t hidden, int6
   binding.bias_gate_up = gate_up_bias;
   binding.bias_down = down_bias;
   ExpertsLaunches launches;
-  if (const int status = make_experts_launches(binding, rows, launches); status != XP_OK) {
+  if (const int status = make_experts_launches(binding, rows, rows, launches); status != XP_OK) {
     return status;
   }
   const hipStream_t hip_stream = static_cast<hipStream_t>(stream);
@@ -2509,7 +2521,7 @@ int xp_moe_template_capture(xp_lane_t lane, const xp_moe_layer_desc *desc, int64
   binding.workspace = lane->workspace;
   binding.fault = lane->fault;
   StepChain chain;
-  if (const int status = make_moe_step(placeholder, binding, capacity, chain); status != XP_OK) {
+  if (const int status = make_moe_step(placeholder, binding, capacity, capacity, chain); status != XP_OK) {
     return status;
   }
   auto t = std::make_unique<Template>();
@@ -2518,8 +2530,9 @@ int xp_moe_template_capture(xp_lane_t lane, const xp_moe_layer_desc *desc, int64
   t->intermediate = signature.intermediate;
   t->capacity = capacity;
   t->moe = signature;
-  t->graphs.resize(1);
-  if (const int status = instantiate_graph(t->graphs.front(), chain); status != XP_OK) {
+  t->plan_rows = template_plan_rows(capacity);
+  t->graphs.resize(t->plan_rows.size());
+  if (const int status = instantiate_graph(t->graphs.back(), chain); status != XP_OK) {
     return status;
   }
   insert_template(lane, std::move(t));

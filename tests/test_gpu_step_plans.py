@@ -1,4 +1,4 @@
-"""Dense steps between a template's capacities: the plan each row count takes.
+"""Steps between a template's capacities: the plan each row count takes.
 
 A template of more than 64 rows keeps tile choices for several row counts; replays at a
 tile's edges must agree with fp64 whatever the choice (192 x 256 and 128 x 256 tiles, K splits
@@ -13,6 +13,7 @@ import torch
 
 from crosspool_amd import _native
 from crosspool_amd.agent import FfnAgent
+from crosspool_amd.moe import MoeFfnWeights, MoeLayerSpec, MoeRouterWeights
 from crosspool_amd.weights import DenseFfnWeights
 
 pytestmark = pytest.mark.gpu
@@ -129,3 +130,48 @@ def test_eager_step_runs_in_the_smallest_accepted_workspace(device):
         torch.cuda.synchronize()
         error = (out[slots.long()].double() - expected).norm() / expected.norm()
         assert error <= 2.0**-8
+
+
+# A MoE template keeps expert tiles for several row counts: every tile family below one capacity,
+# against fp64 over the GPU's own routing, and the same bits through graph dispatch.
+@pytest.mark.parametrize("capacity,rows_list", ((1024, (64, 65, 300, 449, 832, 1024)), (2304, (145, 1100, 2304))))
+def test_moe_steps_between_capacities(device, capacity, rows_list):
+    hidden, intermediate, experts, topk = 256, 128, 8, 2
+    generator = torch.Generator(device=device).manual_seed(3)
+
+    def normal(*shape, std=1.0):
+        return (torch.randn(shape, device=device, generator=generator) * std).bfloat16()
+
+    weights = MoeFfnWeights(normal(experts, 2 * intermediate, hidden, std=0.05), normal(experts, hidden, intermediate, std=0.05),
+                            MoeRouterWeights(normal(experts, hidden, std=0.05)))
+    pool = normal(capacity + 8, hidden)
+    slots = torch.randperm(pool.shape[0], device=device).to(torch.int32)
+    x = pool.double()
+    logits = (x @ weights.router.projection.double().t()).bfloat16().double()
+    picked, ids = torch.softmax(logits, 1).sort(dim=1, descending=True, stable=True)
+    picked, ids = picked[:, :topk] / picked[:, :topk].sum(1, keepdim=True), ids[:, :topk]
+    expected = torch.zeros_like(x)
+    for expert in range(experts):
+        projected = (x @ weights.i_proj[expert].double().t()).bfloat16().double()
+        gate, up = projected[:, 0::2], projected[:, 1::2]
+        y = (gate * torch.sigmoid(gate) * up).bfloat16().double() @ weights.o_proj[expert].double().t()
+        expected += y * (picked * (ids == expert)).sum(1, keepdim=True)
+    outputs = {}
+    for graph_dispatch in (False, True):
+        with FfnAgent(device, graph_dispatch=graph_dispatch) as agent:
+            agent.register_moe_layer(instance_index=0, layer_ordinal=0, weights=weights,
+                                     spec=MoeLayerSpec(routed_expert_count=experts, routed_topk=topk))
+            agent.materialize(maximum_row_capacity=capacity)
+            for rows in rows_list + rows_list[:1]:
+                print(f"moe step plan {rows}/{capacity} graph={graph_dispatch}", flush=True)
+                out = torch.zeros_like(pool)
+                agent.execute(instance_index=0, layer_ordinal=0, pool=pool, slots=slots, rows=rows, out_pool=out)
+                agent.check_health()
+                previous = outputs.setdefault(rows, out)
+                assert torch.equal(out.view(torch.int16), previous.view(torch.int16)), "replays differ"
+    for rows, out in outputs.items():
+        live = slots[:rows].long()
+        difference = (out[live].double() - expected[live]).norm(dim=1) / expected[live].norm(dim=1)
+        # Two route roundings, the combine's and flipped activations; a logit at a rounding
+        # boundary may pick another expert in a few rows.
+        assert difference.median() <= 2.0**-7 and (difference > 2.0**-5).float().mean() <= 0.01, f"{rows} rows"
