@@ -204,6 +204,19 @@ def call(name: str, *args: object) -> int:
     return status
 
 
+def current_stream(device_index: int | None = None) -> ctypes.c_void_p:
+    """Handle of torch's current stream on a device (default: the current device).
+
+    The raw handle: ``torch.cuda.current_stream`` builds a Stream object, 1.8 to 2.7 us of every
+    call on MI355X's host against 0.2.
+    """
+
+    import torch
+
+    index = torch.cuda.current_device() if device_index is None else device_index
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(index))
+
+
 def payload_dtype_code(dtype: object) -> int:
     """XP_DTYPE_BF16 / XP_DTYPE_F16 of a payload dtype (torch.bfloat16 / torch.float16)."""
 

@@ -202,18 +202,18 @@ class ExecutorLane:
         rows = slots.numel() if rows is None else rows
         if not 0 < rows <= slots.numel():
             raise ValueError("row count must be positive and covered by the slot ids")
-        current = torch.cuda.current_stream(self.agent.device)
+        current = _native.current_stream(self.agent.device.index).value or 0
         run_on = self.stream if stream is None else stream
         if stream is None:
             # Lane stream: order after the caller's pending work on the current stream.
-            self.stream.wait_stream(current)
+            self.stream.wait_stream(torch.cuda.current_stream(self.agent.device))
         # A handle of 0 is the legacy default stream (torch's default stream).
         stream_handle = ctypes.c_void_p(run_on.cuda_stream)
         _native.call(
             "xp_replay", self.handle, instance_index, layer_ordinal, rows, ctypes.c_void_p(pool.data_ptr()),
             ctypes.c_void_p(out_pool.data_ptr()), pool.shape[0], ctypes.c_void_p(slots.data_ptr()), stream_handle,
         )
-        if run_on.cuda_stream != current.cuda_stream and not torch.cuda.is_current_stream_capturing():
+        if run_on.cuda_stream != current and not torch.cuda.is_current_stream_capturing():
             # (Under an outer stream capture the kernels become graph nodes and the tensors
             # belong to the capturing caller; no event may be recorded or queried for them.)
             self._retain(run_on, (pool, out_pool, slots))

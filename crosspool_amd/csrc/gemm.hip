@@ -543,6 +543,49 @@ GemmChoice refine_dense_choice(const GemmChoice &base, int64_t rows, int64_t n, 
   return base.kind == GemmKind::Tile && rows >= kStepMinRows ? choose_step_tile(base, rows, n, k) : base;
 }
 
+// The tile and K split of a biased projection at `rows` rows (unsplit when `scratch_bytes` has no
+// room for the ranges' sums), and its modelled time.
+GemmChoice choose_extended(int64_t rows, int64_t n, int64_t k, size_t scratch_bytes, double &us) {
+  const int64_t slabs = (k + 63) / 64;
+  GemmChoice best{GemmKind::Tile, 0, k, 1};
+  us = -1.0;
+  for (int variant = 0; variant < kExtendedTileShapes; ++variant) {
+    for (const int64_t splits : kStepSplits) {
+      const int64_t per_range = (slabs + splits - 1) / splits;
+      if (splits > 1 && (per_range < kStepMinSlabs || (splits - 1) * per_range >= slabs ||
+                         static_cast<uint64_t>(splits * rows * n * 4) > scratch_bytes)) {
+        continue;
+      }
+      const GemmChoice choice{GemmKind::Tile, variant, splits > 1 ? per_range * 64 : k, splits};
+      const double cost = step_us(choice, rows, n, k);
+      if (us < 0.0 || cost < us) {
+        best = choice;
+        us = cost;
+      }
+    }
+  }
+  return best;
+}
+
+KernelLaunch make_extended_gemm(const GemmArgs &args, int64_t capacity, bool gated, const GemmChoice &choice) {
+  if (choice.k_split > 1) {
+    return make_gemm(args, capacity, gated, choice).main;  // the ranges' sums
+  }
+  const TileShape &shape = kTileShapes[choice.variant];
+  GemmArgs record = args;
+  record.capacity = capacity;
+  record.k_slice = choice.k_slice;
+  record.k_split = 1;
+  KernelLaunch kernel;
+  kernel.func = args.payload == kPayloadF16 ? ExtendedKernels<F16Payload>::tile(gated, choice.variant)
+                                            : ExtendedKernels<Bf16Payload>::tile(gated, choice.variant);
+  kernel.grid = dim3(static_cast<unsigned>((args.n + shape.bn - 1) / shape.bn),
+                     static_cast<unsigned>((capacity + shape.bm - 1) / shape.bm), 1);
+  kernel.block = dim3(static_cast<unsigned>(64 * shape.waves), 1, 1);
+  kernel.set_args(record);
+  return kernel;
+}
+
 bool split_gather_fusable(int64_t capacity, int64_t n, int64_t k) {
   const GemmChoice choice = choose_gemm(capacity, n, k, false);
   return choice.kind == GemmKind::Split && choice.variant == 1 && k <= kSplitGatherMaxK;

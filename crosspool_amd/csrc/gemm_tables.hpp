@@ -93,9 +93,19 @@ struct GroupedKernels {
   static const void *split(bool gated);
 };
 
+// The tile shapes of kTileShapes 0 to 3 with the EXTENDED epilogue, without a K split: a biased
+// projection (`bias_stride` 0), gated ones with any activation.
+constexpr int kExtendedTileShapes = 4;
+template <class P>
+struct ExtendedKernels {
+  static const void *tile(bool gated, int variant);
+};
+
 extern template struct DenseKernels<Bf16Payload>;
 extern template struct DenseKernels<F16Payload>;
 extern template struct GroupedKernels<Bf16Payload>;
 extern template struct GroupedKernels<F16Payload>;
+extern template struct ExtendedKernels<Bf16Payload>;
+extern template struct ExtendedKernels<F16Payload>;
 
 }  // namespace xp

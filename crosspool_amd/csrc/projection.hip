@@ -496,6 +496,7 @@ struct ProjectionCost {
 };
 constexpr ProjectionCost kProjectionCosts16[] = {{64, 0.33, 0.27}, {128, 1.37, 0.885}};
 constexpr ProjectionCost kProjectionCosts32[] = {{64, 0.72, 0.59}, {128, 2.5, 2.2}};
+constexpr double kProjectionLaunchUs = 4.7;
 constexpr double kProjectionReduceUs = 2.5;
 constexpr double kProjectionPartialBytesPerUs = 16e6;
 constexpr double kProjectionCus = 256.0;
@@ -509,7 +510,7 @@ ProjectionPlan plan_projection(int64_t rows, int64_t n, int64_t k, int element_b
   // Priced at whole 64-row tiles: the choice then changes only with their number, which makes
   // projection_scratch_bytes exact.
   const int64_t whole_plane_bytes = (rows + 63) / 64 * 64 * n * 4;
-  ProjectionPlan best{64, 1, k};
+  ProjectionPlan best{64, 1, k, 0.0};
   double best_us = -1.0;
   for (const ProjectionCost &cost : element_bytes == 4 ? kProjectionCosts32 : kProjectionCosts16) {
     const int64_t tiles = ((rows + cost.tile - 1) / cost.tile) * ((n + cost.tile - 1) / cost.tile);
@@ -527,7 +528,7 @@ ProjectionPlan plan_projection(int64_t rows, int64_t n, int64_t k, int element_b
         us += kProjectionReduceUs + 2.0 * static_cast<double>(ranges * whole_plane_bytes) / kProjectionPartialBytesPerUs;
       }
       if (best_us < 0.0 || us < best_us) {
-        best = {cost.tile, ranges, ranges > 1 ? per_range * slab : k};
+        best = {cost.tile, ranges, ranges > 1 ? per_range * slab : k, kProjectionLaunchUs + us};
         best_us = us;
       }
     }
@@ -570,14 +571,20 @@ ProjectionLaunch make_projection(const ProjectionArgs &args, const ProjectionPla
   launches.main.block = dim3(256, 1, 1);
   launches.main.set_args(record);
   if (plan.ranges > 1) {
-    launches.reduce.func = args.dtype == kDtypeF32   ? reinterpret_cast<const void *>(&projection_reduce_kernel<F32Payload>)
-                           : args.dtype == kDtypeF16 ? reinterpret_cast<const void *>(&projection_reduce_kernel<F16Payload>)
-                                                     : reinterpret_cast<const void *>(&projection_reduce_kernel<Bf16Payload>);
-    launches.reduce.grid = dim3(static_cast<unsigned>((capacity * ((args.n + 3) / 4) + 255) / 256), 1, 1);
-    launches.reduce.block = dim3(256, 1, 1);
-    launches.reduce.set_args(record);
+    launches.reduce = make_projection_reduce(record, capacity);
   }
   return launches;
+}
+
+KernelLaunch make_projection_reduce(const ProjectionArgs &args, int64_t capacity) {
+  KernelLaunch reduce;
+  reduce.func = args.dtype == kDtypeF32   ? reinterpret_cast<const void *>(&projection_reduce_kernel<F32Payload>)
+                : args.dtype == kDtypeF16 ? reinterpret_cast<const void *>(&projection_reduce_kernel<F16Payload>)
+                                          : reinterpret_cast<const void *>(&projection_reduce_kernel<Bf16Payload>);
+  reduce.grid = dim3(static_cast<unsigned>((capacity * ((args.n + 3) / 4) + 255) / 256), 1, 1);
+  reduce.block = dim3(256, 1, 1);
+  reduce.set_args(args);
+  return reduce;
 }
 
 KernelLaunch make_activation(const ActivationLaunchArgs &args) {

@@ -1416,12 +1416,50 @@ int activation_record(const xp_activation_desc *desc, ActivationArgs &out) {
 
 }  // namespace
 
+namespace {
+
+// 16-bit projections of whole 16-byte rows take the tuned kernels of gemm.hip: without a bias and
+// with no activation or the gated SiLU any of them, otherwise (a bias, another gated activation)
+// the tile kernels' EXTENDED epilogue where their model is below the general kernel's.  The
+// choice is made at the row count rounded up, as a template's for its capacity, so that a
+// workspace for a capacity serves it at every smaller one.
+bool tuned_projection_shape(int64_t n, int64_t k, int dtype) {
+  return dtype_bytes(dtype) == 2 && k % 8 == 0 && n % 16 == 0 && k <= kMaxIntermediate && n <= kMaxIntermediate;
+}
+
+int64_t tuned_projection_rows(int64_t rows) {
+  return rows <= 8 ? 8 : rows <= 16 ? 16 : rows <= 32 ? 32 : (rows + 63) / 64 * 64;
+}
+
+// Below this many rows a biased projection stays on the general kernel.
+constexpr int64_t kExtendedMinRows = 65;
+
+GemmChoice choose_tuned_projection(int64_t capacity, int64_t n, int64_t k, bool gated) {
+  return refine_dense_choice(choose_gemm(capacity, n, k, gated), capacity, n, k);
+}
+
+}  // namespace
+
 size_t xp_projection_workspace_bytes(int64_t rows, int64_t n, int64_t k, int dtype) {
   const size_t element = dtype_bytes(dtype);
   if (rows <= 0 || n <= 0 || k <= 0 || element == 0) {
     return 0;
   }
-  return projection_scratch_bytes(rows, n, k, static_cast<int>(element));
+  size_t most = projection_scratch_bytes(rows, n, k, static_cast<int>(element));
+  if (!tuned_projection_shape(n, k, dtype)) {
+    return most;
+  }
+  for (int64_t capacity = 8; capacity <= tuned_projection_rows(rows); capacity += capacity < 64 ? capacity : 64) {
+    for (const bool gated : {false, true}) {
+      most = std::max(most, gemm_scratch_bytes(choose_tuned_projection(capacity, n, k, gated), capacity, n, k));
+    }
+    if (capacity >= kExtendedMinRows) {
+      double us = 0.0;
+      most = std::max(most, gemm_scratch_bytes(choose_extended(capacity, n, k, static_cast<size_t>(INT64_MAX), us),
+                                               capacity, n, k));
+    }
+  }
+  return most;
 }
 
 int xp_projection(const void *x, int64_t rows, int64_t k, const void *w, int64_t n, const float *bias, void *out,
@@ -1456,8 +1494,48 @@ int xp_projection_split(const void *x, int64_t rows, int64_t k, const void *w, i
   args.n = n;
   args.k = k;
   args.dtype = dtype;
-  const ProjectionPlan plan =
-      plan_projection(rows, n, k, static_cast<int>(element), workspace != nullptr ? workspace_bytes : 0);
+  const size_t scratch_bytes = workspace != nullptr ? workspace_bytes : 0;
+  const ProjectionPlan plan = plan_projection(rows, n, k, static_cast<int>(element), scratch_bytes);
+  if (tuned_projection_shape(n, k, dtype) && aligned16(x) && aligned16(w) && aligned16(out) &&
+      (args.act.gated || args.act.function == kActivationNone)) {
+    const bool gated = args.act.gated != 0;
+    const int64_t capacity = tuned_projection_rows(rows);
+    GemmArgs gemm{};
+    gemm.x = static_cast<const uint16_t *>(x);
+    gemm.w = static_cast<const uint16_t *>(w);
+    gemm.out = static_cast<uint16_t *>(out);
+    gemm.ldx = k;
+    gemm.ldo = gated ? n / 2 : n;
+    gemm.rows = rows;
+    gemm.out_rows = rows;
+    gemm.n = n;
+    gemm.k = k;
+    gemm.act = gated ? GatedSilu{args.act.alpha, args.act.has_limit ? args.act.limit : 0.0f, args.act.up_offset,
+                                 args.act.function, args.act.approximate_tanh}
+                     : default_activation();
+    gemm.payload = dtype == XP_DTYPE_F16 ? kPayloadF16 : kPayloadBf16;
+    gemm.partials = static_cast<float *>(workspace);
+    gemm.bias = bias;
+    const hipStream_t hip_stream = static_cast<hipStream_t>(stream);
+    if (bias == nullptr && (!gated || args.act.function == kActivationSilu)) {
+      const GemmChoice choice = choose_tuned_projection(capacity, n, k, gated);
+      if (gemm_scratch_bytes(choice, capacity, n, k) <= scratch_bytes) {
+        return launch_gemm(make_gemm(gemm, capacity, gated, choice), hip_stream);
+      }
+    } else if (rows >= kExtendedMinRows) {
+      double us = 0.0;
+      const GemmChoice choice = choose_extended(capacity, n, k, scratch_bytes, us);
+      if (us < plan.us) {
+        XP_HIP_CHECK(launch(make_extended_gemm(gemm, capacity, gated, choice), hip_stream));
+        if (choice.k_split > 1) {
+          args.partials = gemm.partials;
+          args.k_slice = choice.k_slice;
+          XP_HIP_CHECK(launch(make_projection_reduce(args, rows), hip_stream));
+        }
+        return XP_OK;
+      }
+    }
+  }
   args.partials = plan.ranges > 1 ? static_cast<float *>(workspace) : nullptr;
   const ProjectionLaunch kernels = make_projection(args, plan, rows, dtype);
   XP_HIP_CHECK(launch(kernels.main, static_cast<hipStream_t>(stream)));

@@ -309,6 +309,7 @@ struct ProjectionPlan {
   int tile;
   int64_t ranges;
   int64_t k_slice;
+  double us = 0.0;  // modelled time
 };
 ProjectionPlan plan_projection(int64_t rows, int64_t n, int64_t k, int element_bytes, size_t scratch_bytes);
 // The most scratch plan_projection uses at any row count up to `capacity`.
@@ -323,6 +324,9 @@ struct ProjectionLaunch {
 // Grids for `capacity` rows.  x_dtype: the tokens' dtype, args.dtype except for 16-bit tokens
 // against fp32 weights.
 ProjectionLaunch make_projection(const ProjectionArgs &args, const ProjectionPlan &plan, int64_t capacity, int x_dtype);
+// The launch that adds the K ranges' sums in args.partials (args.k_slice columns each) and
+// applies the epilogue.
+KernelLaunch make_projection_reduce(const ProjectionArgs &args, int64_t capacity);
 
 // output [elements] = activation of inputs ([elements] ungated, [rows, 2 width] gated).
 struct ActivationLaunchArgs {
@@ -437,6 +441,11 @@ struct GemmLaunch {
   bool usable = true;  // false: the choice names no launchable kernel (callers fail the call)
   int64_t slices = 1;  // K ranges summed by `reduce` (fp32 partials [slices, rows, n]); 1: none
 };
+// A projection with a bias or another gated activation than SiLU on the tile kernels, for rows
+// and weights of whole 16-byte chunks: the choice and its modelled microseconds, and its launch
+// (with a K split the ranges' sums; projection_reduce adds them).
+GemmChoice choose_extended(int64_t rows, int64_t n, int64_t k, size_t scratch_bytes, double &us);
+KernelLaunch make_extended_gemm(const GemmArgs &args, int64_t capacity, bool gated, const GemmChoice &choice);
 // `fused_gather`: the gate_up of a Dense step whose choose_dense_gate_up decision fused the
 // mailbox gather, or a projection for which split_gather_fusable holds (the kernel variant
 // follows that decision, not whether the argument record already holds slot pointers, so a

@@ -20,8 +20,7 @@ from crosspool_amd.weights import DenseFfnWeights
 
 
 def _stream(stream: torch.cuda.Stream | None = None) -> ctypes.c_void_p:
-    stream = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+    return _native.current_stream() if stream is None else ctypes.c_void_p(stream.cuda_stream)
 
 
 def _ptr(tensor: torch.Tensor | None) -> ctypes.c_void_p | None:

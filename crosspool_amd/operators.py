@@ -40,7 +40,7 @@ _ORDER_CODES = {GateUpOrder.CONCATENATED: _native.XP_GATE_UP_CONCATENATED,
 
 
 def _stream() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return _native.current_stream()
 
 
 def _ptr(tensor: torch.Tensor | None) -> ctypes.c_void_p | None:

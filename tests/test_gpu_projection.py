@@ -122,3 +122,45 @@ def test_router_fp32_logits(device, precision, dtype, rows, capacity, hidden, ex
     assert torch.equal(router.ids[:rows].cpu().long(), order[:, :4])
     torch.testing.assert_close(router.weights[:rows].cpu(), scores[:, :4] / scores[:, :4].sum(1, keepdim=True), rtol=1e-5,
                                atol=1e-6)
+
+
+# 16-bit projections of whole 16-byte rows, which the tuned kernels serve: every epilogue, with
+# and without the workspace, around the decode sizes and the tiles.
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))
+@pytest.mark.parametrize("epilogue", ("none", "bias", "silu", "bias+silu", "gelu", "bias+gelu"))
+def test_aligned_projections(device, dtype, epilogue):
+    gated = epilogue not in ("none", "bias")
+    for rows, k, n in ((1, 64, 16), (8, 1000, 528), (9, 2048, 2064), (17, 4096, 272), (33, 512, 1040), (65, 64, 32),
+                       (130, 2048, 2064), (257, 1000, 4112), (300, 6144, 272), (520, 4096, 528)):
+        print(f"aligned projection {dtype} {epilogue} {rows}x{n}x{k}", flush=True)
+        x, w, bias, _ = _operands(device, rows, k, n, dtype)
+        w.mul_(k**-0.5)
+        bias = bias if "bias" in epilogue else None
+        desc = None
+        if gated:
+            desc = _native.ActivationDesc()
+            desc.function = _native.XP_ACTIVATION_GELU if "gelu" in epilogue else _native.XP_ACTIVATION_SILU
+            desc.approximate_tanh, desc.alpha, desc.gated = int("gelu" in epilogue), 1.0, 1
+            desc.has_limit, desc.limit, desc.up_offset = 1, 3.0, 0.5
+        projected = x.double() @ w.double().t() + (0.0 if bias is None else bias.double())
+        if gated:
+            rounded = projected.to(dtype).double()
+            gate, up = rounded[:, 0::2].clamp(max=3.0), rounded[:, 1::2].clamp(-3.0, 3.0)
+            act = torch.nn.functional.gelu(gate, approximate="tanh") if "gelu" in epilogue else gate * torch.sigmoid(gate)
+            expected = act * (up + 0.5)
+        nbytes = _native.library().xp_projection_workspace_bytes(rows, n, k, CODES[dtype])
+        workspace = torch.empty(max(nbytes, 16), device=device, dtype=torch.uint8)
+        for size in sorted({0, nbytes}):
+            out = torch.full((rows, n // 2 if gated else n), 7.0, device=device, dtype=dtype)
+            _native.call(
+                "xp_projection_split", _pointer(x), rows, k, _pointer(w), n, _pointer(bias), _pointer(out), CODES[dtype],
+                None if desc is None else ctypes.byref(desc), _pointer(workspace) if size else None, size,
+                ctypes.c_void_p(torch.cuda.current_stream().cuda_stream),
+            )
+            torch.cuda.synchronize()
+            if gated:
+                # One rounding of the output and the few activations whose input rounds the other way.
+                error = (out.double() - expected).norm() / expected.norm()
+                assert error <= 2.0 ** -(MANTISSA[dtype] + 1), f"{rows}x{n}x{k} workspace {size}: {error:.2e}"
+            else:
+                _assert_within_bound(out, x, w, bias)
