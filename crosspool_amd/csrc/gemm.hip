@@ -430,18 +430,19 @@ GemmChoice choose_step_tile(const GemmChoice &base, int64_t rows, int64_t n, int
     return base;
   }
   double best_us = base_us * (1.0 - kStepGain);
-  auto consider = [&](const GemmChoice &choice) {
-    const double us = step_us(choice, rows, n, k);
-    if (us < best_us) {
-      best = choice;
-      best_us = us;
-    }
-  };
+  const double stream = 2.0 * static_cast<double>(n) * static_cast<double>(k) / kStepWeightBytesPerUs;
+  const double plane_us = 8.0 * static_cast<double>(rows * n) / kStepPartialBytesPerUs;
   for (const StepTile &tile : kStepTiles) {
     for (const int64_t splits : kStepSplits) {
       const int64_t per_range = (slabs + splits - 1) / splits;
-      if (splits == 1 || (per_range >= kStepMinSlabs && (splits - 1) * per_range < slabs)) {  // none empty
-        consider({GemmKind::Tile, tile.variant, splits > 1 ? per_range * 64 : k, splits});
+      if (splits > 1 && (per_range < kStepMinSlabs || (splits - 1) * per_range >= slabs)) {
+        continue;  // ranges too short, or the last one empty
+      }
+      const double us = kStepLaunchUs + stream + step_compute_us(tile, rows, n, per_range, splits) +
+                        (splits > 1 ? kStepReduceUs + static_cast<double>(splits) * plane_us : 0.0);
+      if (us < best_us) {
+        best = {GemmKind::Tile, tile.variant, splits > 1 ? per_range * 64 : k, splits};
+        best_us = us;
       }
     }
     // A first launch of nearly whole rounds, and the remaining columns in a second one.
@@ -453,11 +454,19 @@ GemmChoice choose_step_tile(const GemmChoice &base, int64_t rows, int64_t n, int
       if (weight_tiles == 0 || idle * 12 > kComputeUnits) {
         continue;
       }
-      GemmChoice choice{GemmKind::Tile, tile.variant, k, 1};
-      choice.tail_columns = n - weight_tiles * shape.bn;
+      const int64_t n1 = weight_tiles * shape.bn;
+      const double first = kStepLaunchUs + stream + step_compute_us(tile, rows, n1, slabs, 1);
+      if (kStepTailScale * first + kStepTailUs >= best_us) {
+        break;  // and so do more rounds of this shape
+      }
       for (const StepTile &other : kStepTiles) {
-        choice.tail_variant = other.variant;
-        consider(choice);
+        const double us = kStepTailScale * (first + step_compute_us(other, rows, n - n1, slabs, 1)) + kStepTailUs;
+        if (us < best_us) {
+          best = {GemmKind::Tile, tile.variant, k, 1};
+          best.tail_variant = other.variant;
+          best.tail_columns = n - n1;
+          best_us = us;
+        }
       }
     }
   }

@@ -82,8 +82,9 @@ DensePlan refine_plan(const DensePlan &base, int64_t rows, int64_t hidden, int64
   return plan;
 }
 
-// A template of more than 64 rows holds a plan per kPlanSteps-th of its capacity (at least 64
-// rows apart, one token tile), and a replay takes the smallest that covers its live rows: the
+// A template of more than 64 rows holds plans for the upper half of its capacity, kPlanSteps-ths of
+// it (at least 64 rows, one token tile) apart, and a replay takes the smallest that covers its
+// live rows: the
 // tile shapes, K splits and column splits then suit what runs rather than up to twice as
 // many rows.  Layers at 517 rows of a 1024-row template: Qwen3-4B 158 -> 117 us, 8B 222 -> 184,
 // 1.7B 75 -> 61, the 32B TP shard 93 -> 79; over 23 row counts from 100 to 4000 and six shapes
@@ -99,7 +100,9 @@ int64_t plan_row_step(int64_t capacity) {
 std::vector<int64_t> template_plan_rows(int64_t capacity) {
   std::vector<int64_t> plans;
   const int64_t step = plan_row_step(capacity);
-  for (int64_t rows = step; rows < capacity; rows += step) {
+  // Half the capacity is the next smaller template's (capacities are powers of two): fewer rows
+  // share the first plan above it.
+  for (int64_t rows = capacity / 2 / step * step + step; rows < capacity; rows += step) {
     plans.push_back(rows);
   }
   plans.push_back(capacity);
