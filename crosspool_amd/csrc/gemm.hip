@@ -663,8 +663,9 @@ GemmLaunch make_gemm(const GemmArgs &args, int64_t capacity, bool gated, GemmCho
   const bool f16 = args.payload == kPayloadF16;
   auto tile_kernel = [&](int variant) {
     const WeightLoads loads = capacity > kTileShapes[variant].bm ? WeightLoads::Shared
-                              : args.k % kRotatedPitch == 0 && choice.k_split == 1 ? WeightLoads::StreamRotated
-                                                                                   : WeightLoads::Stream;
+                              : args.k % kRotatedPitch == 0 && choice.k_split <= kRotatedRanges
+                                  ? WeightLoads::StreamRotated
+                                  : WeightLoads::Stream;
     return f16 ? DenseKernels<F16Payload>::tile(gated, variant, loads) : DenseKernels<Bf16Payload>::tile(gated, variant, loads);
   };
   GemmArgs record = args;

@@ -65,6 +65,13 @@ constexpr int kGroupedSplitDepth = 2;
 enum class WeightLoads : int { Shared = 0, Stream = 1, StreamRotated = 2 };
 constexpr int kRotatedTileRows = 128;
 constexpr int64_t kRotatedPitch = 4096;  // columns
+// K ranges start a K split's workgroups at different slabs already: up to four ranges gain from
+// the rotation, eight are even and sixteen lose.  Layers at 17 / 32 / 45 / 64 / 90 / 128 rows: hidden
+// 8192, intermediate 4096 (gate_up in 4 ranges, down in 4 or 2) 58.8 / 60.1 / 61.2 / 63.0 / 68.9 /
+// 77.4 -> 55.3 / 56.6 / 57.5 / 59.3 / 62.0 / 71.8 us; Qwen3-8B (down in 8) 67.8 / 71.9 / 67.6 /
+// 70.6 / 78.8 / 85.4 against 68.0 / 72.0 / 67.7 / 70.7 / 78.5 / 84.4 with it; 1024 / 4096 (down in 16)
+// 22.6 / 23.8 / 24.6 / 25.3 against 22.8 / 24.1 / 24.9 / 25.5 up to 64 rows.
+constexpr int64_t kRotatedRanges = 4;
 
 template <class P>
 struct DenseKernels {

@@ -46,6 +46,7 @@ def _expected(rows, gate_up, down, norm):
         (1536, 8960, 512, (192, 193, 320, 321)),      # 70 weight tiles of 256
         (5120, 3200, 2048, (1025, 1152, 2048)),       # 25 weight tiles, column splits
         (4096, 1032, 128, (33, 64, 65, 128)),         # rotated weight streams, ragged N
+        (8192, 4096, 128, (17, 33, 64, 65, 128)),     # the same over K ranges
         (8192, 264, 64, (33, 64)),                    # the same at another multiple of 8 KB
         (1032, 1000, 300, (65, 128, 129, 300)),       # ragged K and N, a capacity between two steps
         (2048, 6144, 1024, (600, 640, 641)),          # 128 x 256 gate_up
