@@ -502,14 +502,20 @@ __global__ __launch_bounds__(64 * kSplitWaves) void split_gemm_kernel(GemmArgs a
 // by the norm weights (while staging) and the K-range partial sums (after each unit).
 constexpr int kSplitGatheredScratchBytes = (kSplitWaves - 1) * 2 * 64 * 16;
 
-// The gated epilogue of the grouped MoE projections: SiLU exactly as the Dense kernels
-// evaluate it (gated_silu_payload), or ReLU (NaN kept) / GELU (erf or tanh) of the rounded
-// Gate, as compute_gated does (operators/activation.py:19-51), times the rounded Up plus
-// the offset, with the same clipping.
-template <class P, bool CLIP>
+// The gated epilogue of the EXTENDED tile kernels and of the grouped MoE projections: SiLU,
+// ReLU (NaN kept) or GELU (erf or tanh) of the rounded Gate, as compute_gated does
+// (operators/activation.py:19-51), times the rounded Up plus the offset, with the same
+// clipping.  SiLU is evaluated as the Dense kernels evaluate it (gated_silu_payload), or with
+// IEEE_SILU as the general projection and the standalone activation do (expf and an IEEE
+// divide: worst relative error 2.3e-7 over [-30, 30] against 1.8e-6 for rcp and __expf), so
+// that an operator layer's projections agree whichever kernel its row count takes.
+template <class P, bool CLIP, bool IEEE_SILU = false>
 __device__ __forceinline__ float moe_gated_payload(float gate, float up, const GatedSilu &act) {
-  if (act.function != kActivationRelu && act.function != kActivationGelu) {
-    return gated_silu_payload<P, CLIP>(gate, up, act);
+  const bool silu = act.function != kActivationRelu && act.function != kActivationGelu;
+  if constexpr (!IEEE_SILU) {
+    if (silu) {
+      return gated_silu_payload<P, CLIP>(gate, up, act);
+    }
   }
   const uint32_t both = P::pack2(gate, up);
   float g = P::widen(both & 0xffffu);
@@ -519,7 +525,9 @@ __device__ __forceinline__ float moe_gated_payload(float gate, float up, const G
     u = fminf(fmaxf(u, -act.limit), act.limit);
   }
   float f;
-  if (act.function == kActivationRelu) {
+  if (silu) {
+    f = g / (1.0f + expf(-act.alpha * g));
+  } else if (act.function == kActivationRelu) {
     f = (g > 0.0f || g != g) ? g : 0.0f;
   } else if (act.approximate_tanh != 0) {
     f = 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
@@ -1785,9 +1793,10 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs &a, const f32x16 (&
   // Chunk c of row r sits at physical chunk c ^ ((r / 4) % CPR): the two row groups one
   // write instruction covers (rows r and r + 4) then fall in different banks.
   auto slot_of = [](int row, int chunk) { return row * OUT_N + ((chunk ^ ((row >> 2) & (CPR - 1))) << 3); };
-  // EXTENDED (grouped projections with a bias or a ReLU / GELU activation): the expert's
-  // fp32 bias, indexed by weight row (gate_up: Gate and Up of output column c are weight
-  // rows 2 c and 2 c + 1), and the first output column of this wave's tile.
+  // EXTENDED (grouped projections with a bias or a ReLU / GELU activation, and the operator
+  // layer's projections with a bias or a gated activation): the fp32 bias (the expert's),
+  // indexed by weight row (gate_up: Gate and Up of output column c are weight rows 2 c and
+  // 2 c + 1), and the first output column of this wave's tile.
   const float *bias = nullptr;
   int64_t bias_col0 = 0;
   if constexpr (EXTENDED) {
@@ -1819,7 +1828,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs &a, const f32x16 (&
               gate += bias[2 * c];
               up += bias[2 * c + 1];
             }
-            value = moe_gated_payload<P, decltype(clip)::value>(gate, up, a.act);
+            value = moe_gated_payload<P, decltype(clip)::value, !GROUPED>(gate, up, a.act);
           } else if constexpr (GATED) {
             value = gated_silu_payload<P, decltype(clip)::value>(acc[mt][nt][r], acc[mt][nt + NT / 2][r], a.act);
           } else if constexpr (EXTENDED) {

@@ -1421,11 +1421,12 @@ int activation_record(const xp_activation_desc *desc, ActivationArgs &out) {
 
 namespace {
 
-// 16-bit projections of whole 16-byte rows take the tuned kernels of gemm.hip: without a bias and
-// with no activation or the gated SiLU any of them, otherwise (a bias, another gated activation)
-// the tile kernels' EXTENDED epilogue where their model is below the general kernel's.  The
-// choice is made at the row count rounded up, as a template's for its capacity, so that a
-// workspace for a capacity serves it at every smaller one.
+// 16-bit projections of whole 16-byte rows take the tuned kernels of gemm.hip: without a bias or
+// an activation any of them, otherwise (a bias, a gated activation) the tile kernels' EXTENDED
+// epilogue where their model is below the general kernel's.  A gated SiLU without a bias is among
+// the latter: the Dense kernels' own epilogue evaluates it with rcp and __expf, which this entry
+// point's callers have not chosen.  The choice is made at the row count rounded up, as a
+// template's for its capacity, so that a workspace for a capacity serves it at every smaller one.
 bool tuned_projection_shape(int64_t n, int64_t k, int dtype) {
   return dtype_bytes(dtype) == 2 && k % 8 == 0 && n % 16 == 0 && k <= kMaxIntermediate && n <= kMaxIntermediate;
 }
@@ -1434,11 +1435,11 @@ int64_t tuned_projection_rows(int64_t rows) {
   return rows <= 8 ? 8 : rows <= 16 ? 16 : rows <= 32 ? 32 : (rows + 63) / 64 * 64;
 }
 
-// Below this many rows a biased projection stays on the general kernel.
+// Below this many rows a projection with an epilogue stays on the general kernel.
 constexpr int64_t kExtendedMinRows = 65;
 
-GemmChoice choose_tuned_projection(int64_t capacity, int64_t n, int64_t k, bool gated) {
-  return refine_dense_choice(choose_gemm(capacity, n, k, gated), capacity, n, k);
+GemmChoice choose_tuned_projection(int64_t capacity, int64_t n, int64_t k) {
+  return refine_dense_choice(choose_gemm(capacity, n, k, false), capacity, n, k);
 }
 
 }  // namespace
@@ -1453,9 +1454,7 @@ size_t xp_projection_workspace_bytes(int64_t rows, int64_t n, int64_t k, int dty
     return most;
   }
   for (int64_t capacity = 8; capacity <= tuned_projection_rows(rows); capacity += capacity < 64 ? capacity : 64) {
-    for (const bool gated : {false, true}) {
-      most = std::max(most, gemm_scratch_bytes(choose_tuned_projection(capacity, n, k, gated), capacity, n, k));
-    }
+    most = std::max(most, gemm_scratch_bytes(choose_tuned_projection(capacity, n, k), capacity, n, k));
     if (capacity >= kExtendedMinRows) {
       double us = 0.0;
       most = std::max(most, gemm_scratch_bytes(choose_extended(capacity, n, k, static_cast<size_t>(INT64_MAX), us),
@@ -1520,10 +1519,10 @@ int xp_projection_split(const void *x, int64_t rows, int64_t k, const void *w, i
     gemm.partials = static_cast<float *>(workspace);
     gemm.bias = bias;
     const hipStream_t hip_stream = static_cast<hipStream_t>(stream);
-    if (bias == nullptr && (!gated || args.act.function == kActivationSilu)) {
-      const GemmChoice choice = choose_tuned_projection(capacity, n, k, gated);
+    if (bias == nullptr && !gated) {
+      const GemmChoice choice = choose_tuned_projection(capacity, n, k);
       if (gemm_scratch_bytes(choice, capacity, n, k) <= scratch_bytes) {
-        return launch_gemm(make_gemm(gemm, capacity, gated, choice), hip_stream);
+        return launch_gemm(make_gemm(gemm, capacity, false, choice), hip_stream);
       }
     } else if (rows >= kExtendedMinRows) {
       double us = 0.0;

@@ -164,3 +164,43 @@ def test_aligned_projections(device, dtype, epilogue):
                 assert error <= 2.0 ** -(MANTISSA[dtype] + 1), f"{rows}x{n}x{k} workspace {size}: {error:.2e}"
             else:
                 _assert_within_bound(out, x, w, bias)
+
+
+# A SiLU epilogue is evaluated with expf and an IEEE divide whichever kernel the row count, the
+# bias and the workspace choose.  Every row of x is a unit vector, so the projected values are the
+# weights themselves and only the activation and the store round (alpha is a power of two).  The
+# activation's fp32 steps (expf within one ulp, one addition, one division, one product, half an
+# ulp each) leave at most 2.5 x 2^-24 of an output, so it rounds the other way only within that of
+# a tie: a share of at most 2 x 2.5 x 2^-24 of one spacing, which is at least 2^-m / 2 of the
+# output.  (rcp and __expf are several times further off at these Gates, where the product with
+# log2(e) has lost bits.)
+@pytest.mark.parametrize("dtype,alpha,gates,ups", ((torch.bfloat16, 1.0, (-86.0, -40.0), (1.0, 2.0)),
+                                                   (torch.float16, 2.0**-11, (-60000.0, -50000.0), (30000.0, 60000.0))))
+@pytest.mark.parametrize("biased", (False, True))
+@pytest.mark.parametrize("rows", (8, 64, 65, 256))
+def test_silu_epilogues_are_evaluated_in_full_precision(device, dtype, alpha, gates, ups, biased, rows):
+    print(f"silu epilogue {dtype} biased={biased} {rows} rows", flush=True)
+    k, n = 1024, 16384
+    generator = torch.Generator(device=device).manual_seed(rows)
+    w = torch.empty((n, k), device=device, dtype=dtype)
+    for offset, (low, high) in enumerate((gates, ups)):
+        w[offset::2] = (low + (high - low) * torch.rand((n // 2, k), device=device, generator=generator)).to(dtype)
+    x = torch.eye(k, device=device, dtype=dtype)[:rows].contiguous()
+    bias = torch.zeros(n, device=device) if biased else None
+    desc = _native.ActivationDesc()
+    desc.function, desc.alpha, desc.gated = _native.XP_ACTIVATION_SILU, alpha, 1
+    nbytes = _native.library().xp_projection_workspace_bytes(rows, n, k, CODES[dtype])
+    workspace = torch.empty(max(nbytes, 16), device=device, dtype=torch.uint8)
+    gate, up = w[0::2, :rows].cpu().double().t(), w[1::2, :rows].cpu().double().t()
+    expected = (gate / (1.0 + torch.exp(-alpha * gate)) * up).to(dtype)
+    for size in sorted({0, nbytes}):
+        out = torch.empty((rows, n // 2), device=device, dtype=dtype)
+        _native.call(
+            "xp_projection_split", _pointer(x), rows, k, _pointer(w), n, _pointer(bias), _pointer(out), CODES[dtype],
+            ctypes.byref(desc), _pointer(workspace) if size else None, size,
+            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream),
+        )
+        torch.cuda.synchronize()
+        share = (out.cpu() != expected).double().mean().item()
+        bound = 2 * 2.5 * 2.0**-24 / 2.0 ** -(MANTISSA[dtype] + 1)
+        assert share <= bound, f"workspace {size}: share of other roundings {share:.2e} of at most {bound:.2e}"
