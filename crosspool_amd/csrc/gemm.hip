@@ -576,6 +576,13 @@ GemmChoice choose_extended(int64_t rows, int64_t n, int64_t k, size_t scratch_by
   return best;
 }
 
+GemmChoice choose_unsplit(int64_t rows, int64_t n, int64_t k) {
+  double us = 0.0;
+  // The split kernel adds its K ranges in LDS.
+  return rows <= kSplitMaxRows && n * k * 2 <= INT32_MAX ? choose_split(rows, n, k, us)
+                                                          : choose_extended(rows, n, k, 0, us);
+}
+
 KernelLaunch make_extended_gemm(const GemmArgs &args, int64_t capacity, bool gated, const GemmChoice &choice) {
   if (choice.k_split > 1) {
     return make_gemm(args, capacity, gated, choice).main;  // the ranges' sums

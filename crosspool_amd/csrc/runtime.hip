@@ -1629,7 +1629,8 @@ int dense_step_checks(const void *pool_in, const void *pool_out, int64_t pool_ro
 }
 
 // The plan of a step at exactly `rows` rows that fits a workspace of `bytes`: the refined one,
-// else the capacity's own (less scratch).  `needed`: the least bytes that would have served.
+// else the capacity's own.  Either may need more scratch than the other, and more than a larger
+// row count's.  `needed`: the least bytes that would have served.
 bool plan_dense_step(int64_t rows, int64_t hidden, int64_t intermediate, size_t bytes, DensePlan &plan, size_t &needed) {
   const DensePlan base = plan_dense_capacity(rows, hidden, intermediate);
   plan = refine_plan(base, rows, hidden, intermediate);
@@ -1639,6 +1640,18 @@ bool plan_dense_step(int64_t rows, int64_t hidden, int64_t intermediate, size_t 
     needed = std::min(needed, dense_workspace(rows, hidden, intermediate, &plan, 1).bytes);
   }
   return dense_workspace(rows, hidden, intermediate, &plan, 1).bytes <= bytes;
+}
+
+// The same with the projections that leave partial sums replaced by ones that leave none: the
+// step then needs its batch and intermediate regions only.
+void drop_plan_scratch(DensePlan &plan, int64_t hidden, int64_t intermediate) {
+  if (gemm_scratch_bytes(plan.gate_up, plan.rows, 2 * intermediate, hidden) > 0) {
+    plan.gate_up = choose_unsplit(plan.rows, 2 * intermediate, hidden);
+    plan.fused = false;
+  }
+  if (gemm_scratch_bytes(plan.down, plan.rows, hidden, intermediate) > 0) {
+    plan.down = choose_unsplit(plan.rows, hidden, intermediate);
+  }
 }
 
 int run_dense_step(const void *pool_in, void *pool_out, int64_t pool_rows, const int32_t *slots, int64_t rows,
@@ -1685,8 +1698,13 @@ int xp_dense_step(const void *pool_in, void *pool_out, int64_t pool_rows, const 
   XP_REQUIRE(aligned16(workspace), "dense step operands must be 16-byte aligned");
   DensePlan plan{};
   size_t needed = 0;
-  XP_REQUIRE(plan_dense_step(rows, hidden, intermediate, workspace_bytes, plan, needed),
-             "workspace is smaller than xp_dense_workspace_bytes(rows, hidden, intermediate)");
+  // xp_dense_workspace_bytes covers the plans of a capacity; fewer rows can take more K ranges
+  // (4096 x 12288: 160 rows against 256), so a plan that leaves no sums is the last resort.
+  if (!plan_dense_step(rows, hidden, intermediate, workspace_bytes, plan, needed)) {
+    drop_plan_scratch(plan, hidden, intermediate);
+    XP_REQUIRE(dense_workspace(rows, hidden, intermediate, &plan, 1).bytes <= workspace_bytes,
+               "workspace is smaller than the step's gathered batch and intermediate");
+  }
   return run_dense_step(pool_in, pool_out, pool_rows, slots, rows, hidden, intermediate, w_gate_up, w_down,
                         norm_weight, eps, workspace, fault_word, plan, stream);
 }

@@ -423,6 +423,8 @@ GemmChoice choose_gemm(int64_t capacity, int64_t n, int64_t k, bool gated, bool 
 GemmChoice choose_dense_gate_up(int64_t capacity, int64_t n, int64_t k, bool &fused);
 // The choice for `rows` rows of a Dense step whose template's choice is `base`.
 GemmChoice refine_dense_choice(const GemmChoice &base, int64_t rows, int64_t n, int64_t k);
+// The choice for a projection that has no scratch: it leaves no partial sums of K ranges.
+GemmChoice choose_unsplit(int64_t rows, int64_t n, int64_t k);
 // Whether choose_gemm's kernel for an ungated projection at `capacity` rows can take the
 // mailbox gather fused: the split kernel with one token group and K <= 4096 (the MoE step's
 // router projection then gathers and normalises the rows itself).

@@ -199,7 +199,9 @@ int xp_dense_workspace_layout(int64_t capacity, int64_t hidden, int64_t intermed
  * pool_out rows slots[i] (pool_out may equal pool_in).  Same kernels as a replay.  The pool
  * (pool_rows * hidden * 2 bytes) must stay below 2 GiB, the 32-bit buffer range through which
  * the decode kernels gather it (XP_ERROR_INVALID_ARGUMENT otherwise; xp_replay likewise).
- * Replaces Dense.run_into (operators/dense.py:70-86) plus the Transport copies. */
+ * xp_dense_workspace_bytes(capacity) serves every row count up to `capacity`: where `workspace`
+ * has no room for the sums of the K ranges that the row count would take, K is split less or
+ * not at all.  Replaces Dense.run_into (operators/dense.py:70-86) plus the Transport copies. */
 int xp_dense_step(const void *pool_in, void *pool_out, int64_t pool_rows, const int32_t *slots, int64_t rows,
                   int64_t hidden, int64_t intermediate, const void *w_gate_up, const void *w_down,
                   const void *norm_weight, float eps, void *workspace, size_t workspace_bytes, uint32_t *fault_word,

@@ -8,6 +8,8 @@ not divide over the XCDs), repeat bit for bit, and give the same bits through gr
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
@@ -105,32 +107,55 @@ def test_half_block_steps(device, hidden, intermediate, dtype):
             assert error <= (2.0**-8 if dtype is torch.bfloat16 else 2.0**-11), f"{rows} rows: {error:.2e}"
 
 
-def test_eager_step_runs_in_the_smallest_accepted_workspace(device):
-    # The eager step keeps the capacity's own choice where a workspace has no room for the
-    # refined one's K ranges, and refuses only what neither fits.
-    hidden, intermediate, rows = 2560, 9728, 640
+# The eager step keeps the capacity's own choice where a workspace has no room for the refined
+# one's K ranges, takes no K ranges where it has none for either, and refuses only a workspace
+# without room for the batch and the intermediate.
+@pytest.mark.parametrize("rows", (257, 517))
+def test_eager_step_runs_in_the_smallest_accepted_workspace(device, rows):
+    hidden, intermediate = 2560, 9728
+    regions = rows * (hidden + intermediate) * 2
+    scratch = _native.gemm_workspace_bytes(rows, hidden, intermediate, False) + _native.gemm_workspace_bytes(
+        rows, 2 * intermediate, hidden, True)
+    sizes = (_native.dense_workspace_bytes(rows, hidden, intermediate), (regions + 255) // 256 * 256 + scratch, regions)
+    assert sizes[0] > sizes[1] > sizes[2]
+    _check_eager_steps(device, hidden, intermediate, rows, sizes, refused=regions - 16)
+
+
+# A workspace for a capacity serves the row counts below it whose own K ranges would need more.
+@pytest.mark.parametrize("hidden,intermediate,capacity,rows",
+                         ((4096, 12288, 256, 154), (1024, 3072, 128, 72), (5120, 3200, 512, 43), (2048, 6144, 64, 22),
+                          (4096, 12288, 16, 9)))
+def test_eager_step_runs_in_the_workspace_of_a_capacity(device, hidden, intermediate, capacity, rows):
+    _check_eager_steps(device, hidden, intermediate, rows, (_native.dense_workspace_bytes(capacity, hidden, intermediate),
+                                                            rows * (hidden + intermediate) * 2))
+
+
+def _check_eager_steps(device, hidden, intermediate, rows, sizes, refused=None):
     gate_up, down, norm = _layer(device, hidden, intermediate, torch.bfloat16)
     pool = torch.randn((700, hidden), device=device).bfloat16()
     slots = torch.randperm(700, device=device)[:rows].to(torch.int32)
-    base = rows * (hidden + intermediate) * 2
-    scratch = _native.gemm_workspace_bytes(rows, hidden, intermediate, False) + _native.gemm_workspace_bytes(
-        rows, 2 * intermediate, hidden, True)
     expected = _expected(pool[slots.long()], gate_up, down, norm)
-    import ctypes
 
     def pointer(tensor):
         return ctypes.c_void_p(tensor.data_ptr())
 
-    for nbytes in (_native.dense_workspace_bytes(rows, hidden, intermediate), (base + 255) // 256 * 256 + scratch):
-        print(f"eager step workspace {nbytes}", flush=True)
-        workspace = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    def step(nbytes):
+        print(f"eager step {hidden}x{intermediate} {rows} rows workspace {nbytes}", flush=True)
+        workspace = torch.full((nbytes + 256,), 0x7f, dtype=torch.uint8, device=device)
         out = torch.zeros_like(pool)
         _native.call("xp_dense_step", pointer(pool), pointer(out), 700, pointer(slots), rows, hidden, intermediate,
                      pointer(gate_up), pointer(down), pointer(norm), 1e-6, pointer(workspace), nbytes, None,
                      ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
         torch.cuda.synchronize()
+        assert bool((workspace[nbytes:] == 0x7f).all()), "writes outside the workspace"
         error = (out[slots.long()].double() - expected).norm() / expected.norm()
         assert error <= 2.0**-8
+
+    for nbytes in sizes:
+        step(nbytes)
+    if refused is not None:
+        with pytest.raises(_native.NativeError, match="workspace is smaller"):
+            step(refused)
 
 
 # A MoE template keeps expert tiles for several row counts: every tile family below one capacity,

@@ -4,7 +4,8 @@ Covers the Python mirror of the reference interface (capacity buckets,
 workspace geometry, signatures, request metadata, enums) and that the HIP
 library loads and exports every symbol ``include/xpool_amd.h`` declares.  The
 only native calls made are argument-validation paths that return before any
-HIP call, plus pure queries.
+HIP call, plus pure queries (and, without a device only, accepted calls that fail
+at their first launch).
 """
 
 from __future__ import annotations
@@ -194,6 +195,19 @@ def test_dense_step_rejects_mailbox_pools_past_2_gib():
                                       ctypes.c_float(1e-6), None, None)
     assert status == _native.XP_ERROR_INVALID_ARGUMENT
     assert "2 GiB" in _native.last_error()
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="an accepted step would launch on these addresses")
+@pytest.mark.parametrize("hidden,intermediate,capacity", ((4096, 12288, 256), (1024, 3072, 128), (5120, 3200, 512), (2048, 6144, 64)))
+def test_a_capacitys_workspace_serves_every_smaller_step(hidden, intermediate, capacity):
+    # A smaller row count can choose more K ranges than the capacity; the step must then split
+    # less, not refuse.  (Without a device an accepted step fails at its first launch.)
+    nbytes = _native.dense_workspace_bytes(capacity, hidden, intermediate)
+    p = ctypes.c_void_p
+    for rows in range(1, capacity + 1):
+        status = _native.library().xp_dense_step(p(16), p(16), 1 << 10, p(16), rows, hidden, intermediate, p(16), p(16), None,
+                                                 ctypes.c_float(1e-6), p(16), nbytes, None, None)
+        assert status == _native.XP_ERROR_HIP, (rows, _native.last_error())
 
 
 def test_dense_projections_past_one_buffer_range_take_the_tile_kernel():
