@@ -384,6 +384,20 @@ struct xp_agent {
   int live_lanes = 0;
 };
 
+// Lane workspace of a MoE step at `capacity`: the gathered batch, the Router workspace
+// (logits first), routed ids and weights, final ids and weights when shared experts add
+// slots, then the Experts workspace; each region 256-byte aligned.
+struct MoeStepWorkspace {
+  size_t batch;
+  size_t router;
+  size_t routed_ids;
+  size_t routed_weights;
+  size_t final_ids;
+  size_t final_weights;
+  size_t experts;
+  size_t bytes;
+};
+
 // The instantiated hipGraph of one plan.
 struct TemplateGraph {
   hipGraph_t graph = nullptr;
@@ -405,6 +419,7 @@ struct Template {
   std::vector<int64_t> plan_rows;  // increasing; the last is the capacity
   std::vector<DensePlan> plans;    // Dense templates: one per plan_rows
   DenseWorkspace layout{};
+  MoeStepWorkspace moe_layout{};
   // One per plan.  The capacity's is instantiated at capture, the others at their first
   // replay through graph dispatch.
   std::vector<std::unique_ptr<TemplateGraph>> graphs;
@@ -496,6 +511,11 @@ struct RouterWorkspace {
   size_t bytes;
 };
 
+// Where the scratch starts behind the logits.
+size_t router_scratch_offset(int64_t rows, int64_t experts, int precision) {
+  return align_up(static_cast<size_t>(rows * experts) * (precision == XP_ROUTER_PRECISION_PAYLOAD ? 2 : 4), 256);
+}
+
 // PAYLOAD logits go through the Dense projection kernels when their geometry allows it;
 // every other Router projection takes the general one, its fp32 sums kept as the logits (or
 // added by the TopK when K is split).  64 rows x 128 experts x 2048, FP32_LOGITS: 8 us, against
@@ -511,9 +531,8 @@ ProjectionPlan router_projection_plan(int64_t capacity, int64_t hidden, int64_t 
 
 RouterWorkspace router_workspace(int64_t rows, int64_t hidden, int64_t experts, int precision) {
   RouterWorkspace layout{};
-  const bool payload = precision == XP_ROUTER_PRECISION_PAYLOAD;
   layout.logits = 0;
-  layout.scratch = align_up(static_cast<size_t>(rows * experts) * (payload ? 2 : 4), 256);
+  layout.scratch = router_scratch_offset(rows, experts, precision);
   if (router_uses_mfma(hidden, experts, precision)) {
     layout.scratch_bytes = gemm_scratch_bytes(choose_gemm(rows, experts, hidden, false, false), rows, experts, hidden);
   } else {
@@ -599,8 +618,8 @@ bool router_gather_fusable(const xp_moe_layer_desc &d, int64_t capacity) {
 }
 
 RouterLaunches make_router_launches(const RouterBinding &b, int64_t capacity) {
-  const RouterWorkspace layout = router_workspace(capacity, b.hidden, b.experts, b.precision);
-  void *logits = b.workspace + layout.logits;
+  void *logits = b.workspace;
+  float *scratch = reinterpret_cast<float *>(b.workspace + router_scratch_offset(capacity, b.experts, b.precision));
   RouterLaunches launches;
   const float *partials = nullptr;
   int64_t slices = 1;
@@ -620,7 +639,7 @@ RouterLaunches make_router_launches(const RouterBinding &b, int64_t capacity) {
     args.w = static_cast<const uint16_t *>(b.w);
     args.out = static_cast<uint16_t *>(logits);
     args.payload = b.payload;
-    args.partials = layout.scratch_bytes > 0 ? reinterpret_cast<float *>(b.workspace + layout.scratch) : nullptr;
+    args.partials = scratch;
     args.ldx = b.hidden;
     args.ldo = b.experts;
     args.rows = b.rows;
@@ -650,7 +669,7 @@ RouterLaunches make_router_launches(const RouterBinding &b, int64_t capacity) {
     args.dtype = b.precision == XP_ROUTER_PRECISION_FP32 ? kDtypeF32 : payload_dtype;
     const ProjectionPlan plan = router_projection_plan(capacity, b.hidden, b.experts, b.precision);
     if (plan.ranges > 1) {
-      args.partials = reinterpret_cast<float *>(b.workspace + layout.scratch);
+      args.partials = scratch;
       partials = args.partials;
       slices = plan.ranges;
     } else if (b.precision != XP_ROUTER_PRECISION_PAYLOAD) {
@@ -870,20 +889,7 @@ int validate_moe_desc(const xp_moe_layer_desc *d) {
   return payload_kind(d->payload, payload);
 }
 
-// Lane workspace of a MoE step at `capacity`: the gathered batch, the Router workspace
-// (logits first), routed ids and weights, final ids and weights when shared experts add
-// slots, then the Experts workspace; each region 256-byte aligned.
-struct MoeStepWorkspace {
-  size_t batch;
-  size_t router;
-  size_t routed_ids;
-  size_t routed_weights;
-  size_t final_ids;
-  size_t final_weights;
-  size_t experts;
-  size_t bytes;
-};
-
+// The workspace of a MoE template.
 MoeStepWorkspace moe_step_workspace(const xp_moe_layer_desc &d, int64_t capacity) {
   MoeStepWorkspace layout{};
   size_t cursor = 0;
@@ -928,9 +934,9 @@ struct MoeStepBinding {
   uint32_t *fault;
 };
 
-int make_moe_step(const Layer &layer, const MoeStepBinding &b, int64_t capacity, int64_t plan_rows, StepChain &chain) {
+int make_moe_step(const Layer &layer, const MoeStepBinding &b, const MoeStepWorkspace &layout, int64_t capacity,
+                  int64_t plan_rows, StepChain &chain) {
   const xp_moe_layer_desc &d = layer.moe;
-  const MoeStepWorkspace layout = moe_step_workspace(d, capacity);
   uint16_t *batch = reinterpret_cast<uint16_t *>(b.workspace + layout.batch);
   int32_t *routed_ids = reinterpret_cast<int32_t *>(b.workspace + layout.routed_ids);
   float *routed_weights = reinterpret_cast<float *>(b.workspace + layout.routed_weights);
@@ -2066,7 +2072,8 @@ int xp_replay(xp_lane_t lane, int instance_index, int layer_ordinal, int64_t row
     binding.workspace = lane->workspace;
     binding.fault = lane->fault;
     StepChain chain;
-    if (const int status = make_moe_step(layer, binding, selected->capacity, selected->plan_rows[index], chain);
+    if (const int status = make_moe_step(layer, binding, selected->moe_layout, selected->capacity,
+                                         selected->plan_rows[index], chain);
         status != XP_OK) {
       return status;
     }
@@ -2595,10 +2602,10 @@ int xp_moe_template_capture(xp_lane_t lane, const xp_moe_layer_desc *desc, int64
   }
   xp_moe_layer_desc signature = *desc;
   signature.renormalize = desc->renormalize != 0 ? 1 : 0;
-  const size_t needed = moe_step_workspace(signature, capacity).bytes;
-  if (needed > lane->workspace_bytes) {
-    return fail(XP_ERROR_CAPACITY, "Lane workspace is smaller than the template needs (" + std::to_string(needed) +
-                                       " bytes)");
+  const MoeStepWorkspace layout = moe_step_workspace(signature, capacity);
+  if (layout.bytes > lane->workspace_bytes) {
+    return fail(XP_ERROR_CAPACITY, "Lane workspace is smaller than the template needs (" +
+                                       std::to_string(layout.bytes) + " bytes)");
   }
   std::lock_guard<std::mutex> guard(lane->mutex);
   for (const auto &t : lane->templates) {
@@ -2619,7 +2626,7 @@ int xp_moe_template_capture(xp_lane_t lane, const xp_moe_layer_desc *desc, int64
   binding.workspace = lane->workspace;
   binding.fault = lane->fault;
   StepChain chain;
-  if (const int status = make_moe_step(placeholder, binding, capacity, capacity, chain); status != XP_OK) {
+  if (const int status = make_moe_step(placeholder, binding, layout, capacity, capacity, chain); status != XP_OK) {
     return status;
   }
   auto t = std::make_unique<Template>();
@@ -2628,6 +2635,7 @@ int xp_moe_template_capture(xp_lane_t lane, const xp_moe_layer_desc *desc, int64
   t->intermediate = signature.intermediate;
   t->capacity = capacity;
   t->moe = signature;
+  t->moe_layout = layout;
   t->plan_rows = template_plan_rows(capacity);
   t->graphs.resize(t->plan_rows.size());
   if (const int status = instantiate_graph(t->graphs.back(), chain); status != XP_OK) {

@@ -9,12 +9,15 @@ not divide over the XCDs), repeat bit for bit, and give the same bits through gr
 from __future__ import annotations
 
 import ctypes
+import math
+import time
 
 import pytest
 import torch
 
 from crosspool_amd import _native
 from crosspool_amd.agent import FfnAgent
+from crosspool_amd.ffn import RouterProjectionPrecision
 from crosspool_amd.moe import MoeFfnWeights, MoeLayerSpec, MoeRouterWeights
 from crosspool_amd.weights import DenseFfnWeights
 
@@ -201,3 +204,39 @@ def test_moe_steps_between_capacities(device, capacity, rows_list):
         # Two route roundings, the combine's and flipped activations; a logit at a rounding
         # boundary may pick another expert in a few rows.
         assert difference.median() <= 2.0**-7 and (difference > 2.0**-5).float().mean() <= 0.01, f"{rows} rows"
+
+
+def test_moe_replays_prepare_in_the_same_time_at_every_capacity(device):
+    # What follows from the template alone (its workspace, the Router's K ranges) is settled at
+    # capture: the host time of a replay does not grow with the capacity.
+    hidden, intermediate, experts, capacity = 256, 64, 16, 32768
+    generator = torch.Generator(device=device).manual_seed(3)
+
+    def normal(*shape):
+        return torch.randn(shape, device=device, generator=generator) * 0.05
+
+    weights = MoeFfnWeights(normal(experts, 2 * intermediate, hidden).bfloat16(), normal(experts, hidden, intermediate).bfloat16(),
+                            MoeRouterWeights(normal(experts, hidden)))
+    pool = normal(capacity, hidden).bfloat16()
+    slots = torch.arange(capacity, device=device, dtype=torch.int32)
+    out = torch.zeros_like(pool)
+    spec = MoeLayerSpec(routed_expert_count=experts, routed_topk=2, router_projection_precision=RouterProjectionPrecision.FP32)
+    with FfnAgent(device) as agent:
+        agent.register_moe_layer(instance_index=0, layer_ordinal=0, weights=weights, spec=spec)
+        agent.materialize(maximum_row_capacity=capacity)
+
+        def host_us(rows):
+            best = math.inf
+            for _ in range(30):
+                torch.cuda.synchronize()
+                started = time.perf_counter()
+                for _ in range(4):
+                    agent.execute(instance_index=0, layer_ordinal=0, pool=pool, slots=slots, rows=rows, out_pool=out)
+                best = min(best, (time.perf_counter() - started) / 4)
+            torch.cuda.synchronize()
+            return best * 1e6
+
+        small, large = host_us(64), host_us(capacity // 2 + 1)
+        print(f"host us per replay: {small:.1f} at 64 rows, {large:.1f} at {capacity // 2 + 1}", flush=True)
+        # The search over this capacity's row counts, twice a replay, took it from 45 to 96 us.
+        assert large <= 1.5 * small
