@@ -395,6 +395,7 @@ struct MoeStepWorkspace {
   size_t final_ids;
   size_t final_weights;
   size_t experts;
+  size_t router_scratch_bytes;
   size_t bytes;
 };
 
@@ -502,16 +503,10 @@ MoeWorkspace moe_workspace(int64_t rows, int64_t hidden, int64_t intermediate, i
   return layout;
 }
 
-// Router workspace: the logits [rows, experts] (bf16 for the PAYLOAD precision, fp32
-// otherwise), then the PAYLOAD projection's K-slice scratch.
-struct RouterWorkspace {
-  size_t logits;
-  size_t scratch;
-  size_t scratch_bytes;
-  size_t bytes;
-};
-
-// Where the scratch starts behind the logits.
+// Router workspace: the logits [rows, experts] (16-bit for the PAYLOAD precision, fp32
+// otherwise), then as much scratch for the sums of the projection's K ranges as there is: the
+// projection splits K less, or not at all, where the sums of its choice do not fit.  The offset
+// of that scratch:
 size_t router_scratch_offset(int64_t rows, int64_t experts, int precision) {
   return align_up(static_cast<size_t>(rows * experts) * (precision == XP_ROUTER_PRECISION_PAYLOAD ? 2 : 4), 256);
 }
@@ -524,24 +519,26 @@ bool router_uses_mfma(int64_t hidden, int64_t experts, int precision) {
   return precision == XP_ROUTER_PRECISION_PAYLOAD && hidden % 8 == 0 && experts % 8 == 0;
 }
 
-ProjectionPlan router_projection_plan(int64_t capacity, int64_t hidden, int64_t experts, int precision) {
-  return plan_projection(capacity, experts, hidden, precision == XP_ROUTER_PRECISION_FP32 ? 4 : 2,
-                         static_cast<size_t>(INT64_MAX));
+GemmChoice router_choice(int64_t capacity, int64_t hidden, int64_t experts, size_t scratch_bytes) {
+  // (no column split: the Router's launch list has room for one projection kernel)
+  const GemmChoice choice = choose_gemm(capacity, experts, hidden, false, false);
+  return gemm_scratch_bytes(choice, capacity, experts, hidden) <= scratch_bytes ? choice
+                                                                              : choose_unsplit(capacity, experts, hidden);
 }
 
-RouterWorkspace router_workspace(int64_t rows, int64_t hidden, int64_t experts, int precision) {
-  RouterWorkspace layout{};
-  layout.logits = 0;
-  layout.scratch = router_scratch_offset(rows, experts, precision);
+ProjectionPlan router_projection_plan(int64_t capacity, int64_t hidden, int64_t experts, int precision,
+                                      size_t scratch_bytes) {
+  return plan_projection(capacity, experts, hidden, precision == XP_ROUTER_PRECISION_FP32 ? 4 : 2, scratch_bytes);
+}
+
+// Scratch of the choice at `capacity` rows where nothing limits it.
+size_t router_scratch_bytes(int64_t capacity, int64_t hidden, int64_t experts, int precision) {
+  constexpr size_t unlimited = static_cast<size_t>(INT64_MAX);
   if (router_uses_mfma(hidden, experts, precision)) {
-    layout.scratch_bytes = gemm_scratch_bytes(choose_gemm(rows, experts, hidden, false, false), rows, experts, hidden);
-  } else {
-    // For every row count up to `rows`: an operator's workspace serves fewer live rows.
-    layout.scratch_bytes =
-        align_up(projection_scratch_bytes(rows, experts, hidden, precision == XP_ROUTER_PRECISION_FP32 ? 4 : 2), 256);
+    return gemm_scratch_bytes(router_choice(capacity, hidden, experts, unlimited), capacity, experts, hidden);
   }
-  layout.bytes = layout.scratch + layout.scratch_bytes;
-  return layout;
+  const ProjectionPlan plan = router_projection_plan(capacity, hidden, experts, precision, unlimited);
+  return plan.ranges > 1 ? align_up(static_cast<size_t>(plan.ranges * capacity * experts) * 4, 256) : 0;
 }
 
 int validate_router(int64_t experts, int64_t topk, int algorithm, int precision, int weight_rounding) {
@@ -580,7 +577,8 @@ struct RouterBinding {
   const float *correction_bias;
   int32_t *ids;
   float *weights;
-  uint8_t *workspace;  // router_workspace(capacity, ...)
+  uint8_t *workspace;     // the logits, then the scratch at router_scratch_offset(capacity, ...)
+  size_t scratch_bytes;   // room for the sums of K ranges
   int64_t rows;
   int64_t hidden;
   int64_t experts;
@@ -647,9 +645,8 @@ RouterLaunches make_router_launches(const RouterBinding &b, int64_t capacity) {
     args.n = b.experts;
     args.k = b.hidden;
     args.act = default_activation();
-    // (no column split: the Router's launch list has room for one projection kernel)
     const GemmLaunch gemm = make_gemm(args, capacity, false,
-                                      choose_gemm(capacity, b.experts, b.hidden, false, false), b.fused_gather);
+                                      router_choice(capacity, b.hidden, b.experts, b.scratch_bytes), b.fused_gather);
     launches.logits = gemm.main;
     if (gemm.slices > 1) {
       // The TopK adds the K slices itself and stores the logits: no reduction launch (at one
@@ -667,7 +664,8 @@ RouterLaunches make_router_launches(const RouterBinding &b, int64_t capacity) {
     args.k = b.hidden;
     const int payload_dtype = b.payload == kPayloadF16 ? kDtypeF16 : kDtypeBf16;
     args.dtype = b.precision == XP_ROUTER_PRECISION_FP32 ? kDtypeF32 : payload_dtype;
-    const ProjectionPlan plan = router_projection_plan(capacity, b.hidden, b.experts, b.precision);
+    const ProjectionPlan plan =
+        router_projection_plan(capacity, b.hidden, b.experts, b.precision, b.scratch_bytes);
     if (plan.ranges > 1) {
       args.partials = scratch;
       partials = args.partials;
@@ -889,9 +887,9 @@ int validate_moe_desc(const xp_moe_layer_desc *d) {
   return payload_kind(d->payload, payload);
 }
 
-// The workspace of a MoE template.
-MoeStepWorkspace moe_step_workspace(const xp_moe_layer_desc &d, int64_t capacity) {
+MoeStepWorkspace moe_step_workspace(const xp_moe_layer_desc &d, int64_t capacity, size_t router_scratch) {
   MoeStepWorkspace layout{};
+  layout.router_scratch_bytes = router_scratch;
   size_t cursor = 0;
   auto region = [&](size_t bytes) {
     const size_t offset = cursor;
@@ -900,7 +898,7 @@ MoeStepWorkspace moe_step_workspace(const xp_moe_layer_desc &d, int64_t capacity
   };
   const int64_t topk = effective_topk(d);
   layout.batch = region(static_cast<size_t>(capacity * d.hidden) * 2);
-  layout.router = region(router_workspace(capacity, d.hidden, d.routed_experts, d.precision).bytes);
+  layout.router = region(router_scratch_offset(capacity, d.routed_experts, d.precision) + router_scratch);
   layout.routed_ids = region(static_cast<size_t>(capacity * d.routed_topk) * 4);
   layout.routed_weights = region(static_cast<size_t>(capacity * d.routed_topk) * 4);
   if (topk > d.routed_topk) {
@@ -913,6 +911,11 @@ MoeStepWorkspace moe_step_workspace(const xp_moe_layer_desc &d, int64_t capacity
   layout.experts = region(moe_workspace(capacity, d.hidden, d.intermediate, d.experts, topk).bytes);
   layout.bytes = cursor;
   return layout;
+}
+
+// With the scratch the Router's choice at `capacity` rows takes.
+MoeStepWorkspace moe_step_workspace(const xp_moe_layer_desc &d, int64_t capacity) {
+  return moe_step_workspace(d, capacity, router_scratch_bytes(capacity, d.hidden, d.routed_experts, d.precision));
 }
 
 int validate_moe_capacity(const xp_moe_layer_desc &d, int64_t capacity) {
@@ -975,6 +978,7 @@ int make_moe_step(const Layer &layer, const MoeStepBinding &b, const MoeStepWork
   router.ids = routed_ids;
   router.weights = routed_weights;
   router.workspace = b.workspace + layout.router;
+  router.scratch_bytes = layout.router_scratch_bytes;
   router.rows = b.rows;
   router.hidden = d.hidden;
   router.experts = d.routed_experts;
@@ -2323,7 +2327,12 @@ size_t xp_moe_router_workspace_bytes(int64_t rows, int64_t hidden, int64_t exper
   if (rows <= 0 || hidden <= 0 || experts <= 0) {
     return 0;
   }
-  return router_workspace(rows, hidden, experts, precision).bytes;
+  const size_t offset = router_scratch_offset(rows, experts, precision);
+  if (router_uses_mfma(hidden, experts, precision)) {
+    return offset + router_scratch_bytes(rows, hidden, experts, precision);
+  }
+  // For every row count up to `rows`: an operator's workspace serves fewer live rows.
+  return offset + align_up(projection_scratch_bytes(rows, experts, hidden, precision == XP_ROUTER_PRECISION_FP32 ? 4 : 2), 256);
 }
 
 int xp_moe_router_topk(const void *logits, int logits_dtype, int64_t rows, int64_t experts, int64_t topk,
@@ -2378,9 +2387,9 @@ int xp_moe_router(const void *hidden_states, int64_t rows, int64_t hidden, const
              "router pointers must be non-null");
   XP_REQUIRE(!router_uses_mfma(hidden, experts, precision) || (aligned16(hidden_states) && aligned16(router_weights)),
              "router inputs must be 16-byte aligned");
-  const RouterWorkspace layout = router_workspace(rows, hidden, experts, precision);
-  XP_REQUIRE(workspace != nullptr && workspace_bytes >= layout.bytes && aligned16(workspace),
-             "router workspace is missing or smaller than xp_moe_router_workspace_bytes");
+  const size_t scratch_offset = router_scratch_offset(rows, experts, precision);
+  XP_REQUIRE(workspace != nullptr && workspace_bytes >= scratch_offset && aligned16(workspace),
+             "router workspace is missing or smaller than the logits");
   RouterBinding binding{};
   binding.x = static_cast<const uint16_t *>(hidden_states);
   binding.w = router_weights;
@@ -2388,6 +2397,7 @@ int xp_moe_router(const void *hidden_states, int64_t rows, int64_t hidden, const
   binding.ids = ids;
   binding.weights = weights;
   binding.workspace = static_cast<uint8_t *>(workspace);
+  binding.scratch_bytes = workspace_bytes - scratch_offset;
   binding.rows = rows;
   binding.hidden = hidden;
   binding.experts = experts;
@@ -2582,7 +2592,7 @@ int xp_moe_step_workspace_layout(const xp_moe_layer_desc *desc, int64_t capacity
   XP_REQUIRE(offsets != nullptr, "output pointer must be non-null");
   const MoeStepWorkspace layout = moe_step_workspace(*desc, capacity);
   offsets[0] = layout.batch;
-  offsets[1] = layout.router + router_workspace(capacity, desc->hidden, desc->routed_experts, desc->precision).logits;
+  offsets[1] = layout.router;
   offsets[2] = layout.routed_ids;
   offsets[3] = layout.routed_weights;
   offsets[4] = layout.final_ids;
@@ -2602,7 +2612,10 @@ int xp_moe_template_capture(xp_lane_t lane, const xp_moe_layer_desc *desc, int64
   }
   xp_moe_layer_desc signature = *desc;
   signature.renormalize = desc->renormalize != 0 ? 1 : 0;
-  const MoeStepWorkspace layout = moe_step_workspace(signature, capacity);
+  MoeStepWorkspace layout = moe_step_workspace(signature, capacity);
+  if (layout.bytes > lane->workspace_bytes) {
+    layout = moe_step_workspace(signature, capacity, 0);  // a Router that splits no K
+  }
   if (layout.bytes > lane->workspace_bytes) {
     return fail(XP_ERROR_CAPACITY, "Lane workspace is smaller than the template needs (" +
                                        std::to_string(layout.bytes) + " bytes)");

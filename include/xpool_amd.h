@@ -409,7 +409,11 @@ int xp_moe_router_topk(const void *logits, int logits_dtype, int64_t rows, int64
                        int algorithm, const float *correction_bias, int renormalize, int weight_rounding,
                        int32_t *ids, float *weights, xp_stream_t stream);
 
-/* Workspace bytes of xp_moe_router (the logits and the projection's K-slice scratch). */
+/* Workspace bytes of xp_moe_router: the logits and the scratch for the sums of the projection's
+ * K ranges at `rows` rows.  Any workspace that holds the logits (rows x experts values of 2
+ * bytes, 4 with fp32 logits, rounded up to 256) is accepted: K is then split less, so that the
+ * workspace of a capacity serves every smaller row count.  A MoE template likewise accepts a
+ * Lane workspace without that scratch. */
 size_t xp_moe_router_workspace_bytes(int64_t rows, int64_t hidden, int64_t experts, int precision);
 
 /* Router: logits = hidden_states [rows, hidden] . router_weights^T, with hidden_states of

@@ -124,6 +124,30 @@ def test_router_fp32_logits(device, precision, dtype, rows, capacity, hidden, ex
                                atol=1e-6)
 
 
+# A Router splits K as far as its workspace has room for the sums: one that holds the logits
+# only, and one sized for a capacity whose own choice needs less scratch than the live rows'.
+@pytest.mark.parametrize("precision", tuple(RouterProjectionPrecision))
+@pytest.mark.parametrize("rows,capacity,hidden,experts", ((9, 16, 2048, 128), (33, 66, 2048, 128), (639, 640, 2048, 128),
+                                                          (512, 513, 4096, 256), (65, 128, 1003, 130)))
+def test_router_runs_in_smaller_workspaces(device, precision, rows, capacity, hidden, experts):
+    generator = torch.Generator(device=device).manual_seed(rows + hidden)
+    x = torch.randn((capacity, hidden), device=device, generator=generator).bfloat16()
+    weight_dtype = torch.float32 if precision is RouterProjectionPrecision.FP32 else torch.bfloat16
+    w = torch.randn((experts, hidden), device=device, generator=generator).to(weight_dtype)
+    router = Router(row_capacity=capacity, hidden_size=hidden, routed_expert_count=experts, routed_topk=4,
+                    precision=precision, device=device)
+    whole = router.workspace
+    logits = rows * experts * router.logits.element_size()
+    for nbytes in (whole.numel(), (logits + 255) // 256 * 256):
+        print(f"router {precision.name} {rows}/{capacity}x{experts}x{hidden} workspace {nbytes}", flush=True)
+        whole.fill_(0x7f)
+        router.workspace = whole[:nbytes]
+        router.run_into(hidden_states=x, router_weights=MoeRouterWeights(w), rows=rows)
+        torch.cuda.synchronize()
+        _assert_within_bound(router.logits[:rows], x[:rows], w, None)
+        assert bool((whole[nbytes:] == 0x7f).all()), "sums outside the workspace"
+
+
 # 16-bit projections of whole 16-byte rows, which the tuned kernels serve: every epilogue, with
 # and without the workspace, around the decode sizes and the tiles.
 @pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))

@@ -16,7 +16,7 @@ import pytest
 import torch
 
 from crosspool_amd import _native
-from crosspool_amd.agent import FfnAgent
+from crosspool_amd.agent import ExecutorLane, FfnAgent
 from crosspool_amd.ffn import RouterProjectionPrecision
 from crosspool_amd.moe import MoeFfnWeights, MoeLayerSpec, MoeRouterWeights
 from crosspool_amd.weights import DenseFfnWeights
@@ -204,6 +204,48 @@ def test_moe_steps_between_capacities(device, capacity, rows_list):
         # Two route roundings, the combine's and flipped activations; a logit at a rounding
         # boundary may pick another expert in a few rows.
         assert difference.median() <= 2.0**-7 and (difference > 2.0**-5).float().mean() <= 0.01, f"{rows} rows"
+
+
+@pytest.mark.parametrize("precision", (RouterProjectionPrecision.FP32, RouterProjectionPrecision.FP32_LOGITS))
+def test_moe_template_runs_in_a_lane_without_router_scratch(device, precision):
+    hidden, intermediate, experts, topk, capacity = 2048, 64, 128, 4, 256
+    generator = torch.Generator(device=device).manual_seed(3)
+
+    def normal(*shape):
+        return torch.randn(shape, device=device, generator=generator)
+
+    router = normal(experts, hidden) * 0.1
+    router = router if precision is RouterProjectionPrecision.FP32 else router.bfloat16()
+    weights = MoeFfnWeights((normal(experts, 2 * intermediate, hidden) * 0.05).bfloat16(),
+                            (normal(experts, hidden, intermediate) * 0.05).bfloat16(), MoeRouterWeights(router))
+    pool = normal(capacity, hidden).bfloat16()
+    slots = torch.randperm(capacity, device=device, generator=generator).to(torch.int32)
+    with FfnAgent(device) as agent:
+        agent.register_moe_layer(
+            instance_index=0, layer_ordinal=0, weights=weights,
+            spec=MoeLayerSpec(routed_expert_count=experts, routed_topk=topk, router_projection_precision=precision))
+        agent.materialize(maximum_row_capacity=capacity)
+        template = next(t for t in agent.templates.values() if t.signature.payload_row_capacity == capacity)
+        layout = _native.moe_step_workspace_layout(template.signature.native_descriptor(), capacity)
+        scratch = layout[2] - layout[1] - capacity * experts * 4
+        assert scratch > 0
+        print(f"moe lane {precision.name} {layout[7]} less {scratch} bytes", flush=True)
+        lane = ExecutorLane(agent, layout[7] - scratch)
+        lane.capture(template)
+        for rows in (1, 100, capacity):
+            out, expected = torch.zeros_like(pool), torch.zeros_like(pool)
+            lane.replay(instance_index=0, layer_ordinal=0, pool=pool, slots=slots, rows=rows, out_pool=out)
+            agent.execute(instance_index=0, layer_ordinal=0, pool=pool, slots=slots, rows=rows, out_pool=expected)
+            torch.cuda.synchronize()
+            # The Router's fp32 sums in another order: its weights move by a few 2^-24.
+            assert (out.double() - expected.double()).norm() <= 2.0**-8 * expected.double().norm()
+        lane.close()
+        with pytest.raises(_native.NativeError, match="smaller than the template needs"):
+            small = ExecutorLane(agent, layout[7] - scratch - 256)
+            try:
+                small.capture(template)
+            finally:
+                small.close()
 
 
 def test_moe_replays_prepare_in_the_same_time_at_every_capacity(device):
