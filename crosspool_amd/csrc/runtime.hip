@@ -1963,7 +1963,13 @@ int xp_template_capture(xp_lane_t lane, int64_t hidden, int64_t intermediate, in
   }
   XP_REQUIRE(capacity > 0, "template capacity must be positive");
   std::vector<DensePlan> plans = plan_dense_template(capacity, hidden, intermediate);
-  const DenseWorkspace layout = dense_workspace(capacity, hidden, intermediate, plans.data(), plans.size());
+  DenseWorkspace layout = dense_workspace(capacity, hidden, intermediate, plans.data(), plans.size());
+  if (layout.bytes > lane->workspace_bytes) {
+    // The capacity's unrefined plan alone, whose K ranges need less scratch where other row
+    // counts' take more.
+    plans = {plan_dense_capacity(capacity, hidden, intermediate)};
+    layout = dense_workspace(capacity, hidden, intermediate, plans.data(), plans.size());
+  }
   if (layout.bytes > lane->workspace_bytes) {
     return fail(XP_ERROR_CAPACITY, "Lane workspace is smaller than the template needs (" +
                                        std::to_string(layout.bytes) + " bytes)");
@@ -1990,7 +1996,9 @@ int xp_template_capture(xp_lane_t lane, int64_t hidden, int64_t intermediate, in
   t->intermediate = intermediate;
   t->payload = payload;
   t->capacity = capacity;
-  t->plan_rows = template_plan_rows(capacity);
+  for (const DensePlan &plan : plans) {
+    t->plan_rows.push_back(plan.rows);
+  }
   t->plans = std::move(plans);
   t->layout = layout;
   t->graphs.resize(t->plans.size());

@@ -181,9 +181,13 @@ int xp_activation(const void *inputs, void *output, int64_t rows, int64_t width,
  * (src/xpool/runtime/ffnagent/operators/linear.py:111-131). */
 size_t xp_gemm_workspace_bytes(int64_t rows, int64_t n, int64_t k, int gated);
 
-/* Bytes of Lane workspace one Dense step at `capacity` rows needs
- * (gathered batch + activated intermediate + K-slice partial sums).  Replaces DenseExecutionPlan's
- * WorkspaceLayout (src/xpool/runtime/ffnagent/operators/dense.py:24-52). */
+/* Bytes of Lane workspace a Dense template of `capacity` rows asks for: the gathered batch, the
+ * activated intermediate and the partial sums of the K ranges that any of its plans takes (a
+ * plan per sixteenth of the capacity; the sums are 63 of 130 MB for hidden 4096, intermediate
+ * 12288 at 2048 rows, 42 of 55 MB for 8192, 4096 at 512).  xp_template_capture also accepts a
+ * Lane workspace with room for the sums of the capacity's own choice only (none in these two
+ * cases); every replay then takes that choice.  Replaces DenseExecutionPlan's WorkspaceLayout
+ * (src/xpool/runtime/ffnagent/operators/dense.py:24-52). */
 size_t xp_dense_workspace_bytes(int64_t capacity, int64_t hidden, int64_t intermediate);
 
 /* Byte offsets of that workspace's regions: [0] the gathered (normalised) batch

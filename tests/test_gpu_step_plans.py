@@ -161,6 +161,41 @@ def _check_eager_steps(device, hidden, intermediate, rows, sizes, refused=None):
             step(refused)
 
 
+# A Lane whose workspace has no room for the K ranges of the plans between two capacities takes the
+# capacity's own choice at every row count.
+@pytest.mark.parametrize("hidden,intermediate,capacity", ((8192, 4096, 512), (1536, 8960, 512), (4096, 12288, 2048)))
+def test_template_runs_in_a_lane_for_the_capacitys_own_choice(device, hidden, intermediate, capacity):
+    gate_up, down, norm = _layer(device, hidden, intermediate, torch.bfloat16)
+    pool = torch.randn((capacity, hidden), device=device, generator=torch.Generator(device=device).manual_seed(4)).bfloat16()
+    slots = torch.randperm(capacity, device=device).to(torch.int32)
+    regions = capacity * (hidden + intermediate) * 2
+    scratch = _native.gemm_workspace_bytes(capacity, hidden, intermediate, False) + _native.gemm_workspace_bytes(
+        capacity, 2 * intermediate, hidden, True)
+    nbytes = (regions + 255) // 256 * 256 + scratch if scratch else regions
+    assert nbytes < _native.dense_workspace_bytes(capacity, hidden, intermediate)
+    with FfnAgent(device) as agent:
+        agent.register_layer(instance_index=0, layer_ordinal=0, norm_weight=norm, eps=1e-6,
+                             weights=DenseFfnWeights.from_tensors(gate_up, down))
+        agent.materialize(maximum_row_capacity=capacity)
+        template = next(t for t in agent.templates.values() if t.signature.payload_row_capacity == capacity)
+        for graph_dispatch in (False, True):
+            lane = ExecutorLane(agent, nbytes, graph_dispatch=graph_dispatch)
+            lane.capture(template)
+            for rows in (1, capacity // 2 + 1, capacity):
+                print(f"small lane {hidden}x{intermediate} {rows}/{capacity} graph={graph_dispatch}", flush=True)
+                out = torch.zeros_like(pool)
+                lane.replay(instance_index=0, layer_ordinal=0, pool=pool, slots=slots, rows=rows, out_pool=out)
+                lane.synchronize()
+                live = slots[:rows].long()
+                expected = _expected(pool[live], gate_up, down, norm)
+                assert (out[live].double() - expected).norm() <= 2.0**-8 * expected.norm()
+            lane.close()
+        lane = ExecutorLane(agent, nbytes - 256)
+        with pytest.raises(_native.NativeError, match="smaller than the template needs"):
+            lane.capture(template)
+        lane.close()
+
+
 # A MoE template keeps expert tiles for several row counts: every tile family below one capacity,
 # against fp64 over the GPU's own routing, and the same bits through graph dispatch.
 @pytest.mark.parametrize("capacity,rows_list", ((1024, (64, 65, 300, 449, 832, 1024)), (2304, (145, 1100, 2304))))
