@@ -421,8 +421,8 @@ struct Template {
   std::vector<DensePlan> plans;    // Dense templates: one per plan_rows
   DenseWorkspace layout{};
   MoeStepWorkspace moe_layout{};
-  // One per plan.  The capacity's is instantiated at capture, the others at their first
-  // replay through graph dispatch.
+  // One per plan: the capacity's is instantiated at capture, the others there too on a Lane with
+  // graph dispatch, else when it is switched on (instantiate_plans).
   std::vector<std::unique_ptr<TemplateGraph>> graphs;
 };
 
@@ -1162,9 +1162,63 @@ void insert_template(xp_lane *lane, std::unique_ptr<Template> t) {
   });
 }
 
+// The graphs of a template's plans from `first` on that it does not hold yet, so that a replay
+// only rebinds and launches.  The bindings are placeholders: a replay rebinds every argument
+// record.  The caller has made the Lane's device current.
+int instantiate_plans(const xp_lane *lane, Template &t, size_t first) {
+  for (size_t index = first; index < t.graphs.size(); ++index) {
+    if (t.graphs[index] != nullptr) {
+      continue;
+    }
+    StepChain chain;
+    if (t.kind == XP_LAYER_MOE) {
+      Layer placeholder{};
+      placeholder.kind = XP_LAYER_MOE;
+      placeholder.moe = t.moe;
+      placeholder.hidden = t.hidden;
+      placeholder.intermediate = t.intermediate;
+      MoeStepBinding binding{};
+      binding.rows = t.capacity;
+      binding.pool_rows = t.capacity;
+      binding.workspace = lane->workspace;
+      binding.fault = lane->fault;
+      if (const int status = make_moe_step(placeholder, binding, t.moe_layout, t.capacity, t.plan_rows[index], chain);
+          status != XP_OK) {
+        return status;
+      }
+    } else {
+      DenseBinding binding{};
+      binding.hidden = t.hidden;
+      binding.intermediate = t.intermediate;
+      binding.payload = t.payload;
+      binding.rows = 0;
+      binding.workspace = lane->workspace;
+      binding.fault = lane->fault;
+      chain = dense_chain(binding, t.layout, t.plans[index]);
+    }
+    if (const int status = instantiate_graph(t.graphs[index], chain); status != XP_OK) {
+      return status;
+    }
+  }
+  return XP_OK;
+}
+
+// A new template with its graphs, onto the Lane's list.
+int install_template(xp_lane *lane, std::unique_ptr<Template> t) {
+  XP_HIP_CHECK(hipSetDevice(lane->agent->device));
+  t->graphs.resize(t->plan_rows.size());
+  const size_t first = lane->graph_dispatch ? 0 : t->graphs.size() - 1;
+  if (const int status = instantiate_plans(lane, *t, first); status != XP_OK) {
+    destroy_template(*t);
+    return status;
+  }
+  insert_template(lane, std::move(t));
+  return XP_OK;
+}
+
 // Launch a replay's chain: directly on the stream, or (graph dispatch) by rebinding the
 // nodes of its plan's graph whose argument record changed and launching that graph.
-int run_chain(xp_lane *lane, std::unique_ptr<TemplateGraph> &graph, const StepChain &chain, hipStream_t target) {
+int run_chain(xp_lane *lane, const std::unique_ptr<TemplateGraph> &graph, const StepChain &chain, hipStream_t target) {
   if (!chain.usable) {
     return fail(XP_ERROR_INVALID_ARGUMENT, kUnusableChoice);
   }
@@ -1182,9 +1236,7 @@ int run_chain(xp_lane *lane, std::unique_ptr<TemplateGraph> &graph, const StepCh
     return XP_OK;
   }
   if (graph == nullptr) {
-    if (const int status = instantiate_graph(graph, chain); status != XP_OK) {
-      return status;
-    }
+    return fail(XP_ERROR_STATE, "the plan's graph was not instantiated with graph dispatch");
   }
   TemplateGraph &t = *graph;
   if (chain.count != t.node_count) {
@@ -1923,6 +1975,14 @@ int xp_lane_stream(xp_lane_t lane, xp_stream_t *out) {
 int xp_lane_set_graph_dispatch(xp_lane_t lane, int use_graph) {
   XP_REQUIRE(lane != nullptr, "lane must be non-null");
   std::lock_guard<std::mutex> guard(lane->mutex);
+  if (use_graph != 0 && !lane->graph_dispatch) {
+    XP_HIP_CHECK(hipSetDevice(lane->agent->device));
+    for (const auto &t : lane->templates) {
+      if (const int status = instantiate_plans(lane, *t, 0); status != XP_OK) {
+        return status;
+      }
+    }
+  }
   lane->graph_dispatch = use_graph != 0;
   return XP_OK;
 }
@@ -1981,15 +2041,6 @@ int xp_template_capture(xp_lane_t lane, int64_t hidden, int64_t intermediate, in
       return XP_OK;
     }
   }
-  XP_HIP_CHECK(hipSetDevice(lane->agent->device));
-  // Placeholder binding: a replay rebinds every argument record before launching.
-  DenseBinding binding{};
-  binding.hidden = hidden;
-  binding.intermediate = intermediate;
-  binding.payload = payload;
-  binding.rows = 0;
-  binding.workspace = lane->workspace;
-  binding.fault = lane->fault;
   auto t = std::make_unique<Template>();
   t->kind = XP_LAYER_DENSE;
   t->hidden = hidden;
@@ -2001,13 +2052,7 @@ int xp_template_capture(xp_lane_t lane, int64_t hidden, int64_t intermediate, in
   }
   t->plans = std::move(plans);
   t->layout = layout;
-  t->graphs.resize(t->plans.size());
-  if (const int status = instantiate_graph(t->graphs.back(), dense_chain(binding, t->layout, t->plans.back()));
-      status != XP_OK) {
-    return status;
-  }
-  insert_template(lane, std::move(t));
-  return XP_OK;
+  return install_template(lane, std::move(t));
 }
 
 int xp_template_capacities(xp_lane_t lane, int64_t hidden, int64_t intermediate, int payload_dtype,
@@ -2634,22 +2679,6 @@ int xp_moe_template_capture(xp_lane_t lane, const xp_moe_layer_desc *desc, int64
       return XP_OK;
     }
   }
-  XP_HIP_CHECK(hipSetDevice(lane->agent->device));
-  // Placeholder layer and binding: a replay rebinds every argument record before launching.
-  Layer placeholder{};
-  placeholder.kind = XP_LAYER_MOE;
-  placeholder.moe = signature;
-  placeholder.hidden = signature.hidden;
-  placeholder.intermediate = signature.intermediate;
-  MoeStepBinding binding{};
-  binding.rows = capacity;
-  binding.pool_rows = capacity;
-  binding.workspace = lane->workspace;
-  binding.fault = lane->fault;
-  StepChain chain;
-  if (const int status = make_moe_step(placeholder, binding, layout, capacity, capacity, chain); status != XP_OK) {
-    return status;
-  }
   auto t = std::make_unique<Template>();
   t->kind = XP_LAYER_MOE;
   t->hidden = signature.hidden;
@@ -2658,12 +2687,7 @@ int xp_moe_template_capture(xp_lane_t lane, const xp_moe_layer_desc *desc, int64
   t->moe = signature;
   t->moe_layout = layout;
   t->plan_rows = template_plan_rows(capacity);
-  t->graphs.resize(t->plan_rows.size());
-  if (const int status = instantiate_graph(t->graphs.back(), chain); status != XP_OK) {
-    return status;
-  }
-  insert_template(lane, std::move(t));
-  return XP_OK;
+  return install_template(lane, std::move(t));
 }
 
 }  // extern "C"

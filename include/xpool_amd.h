@@ -264,7 +264,8 @@ int xp_lane_clear_fault(xp_lane_t lane);
 int xp_lane_synchronize(xp_lane_t lane);
 /* Replay dispatch of this Lane: 0 (default) launches a template's kernels directly on the
  * stream, nonzero launches its instantiated hipGraph (rebinding only the kernel nodes whose
- * arguments changed).  Both run the same kernels with the same arguments.  No counterpart
+ * arguments changed; switching it on instantiates the graphs of every plan of the Lane's
+ * templates, as a later xp_template_capture does, so that no replay has to).  Both run the same kernels with the same arguments.  No counterpart
  * in the reference, whose CUDA graphs are always launched (runtime.cu:701-1006); on MI355X a
  * hipGraphLaunch adds about 4-5 us of GPU time per Dense replay at decode sizes (measured on
  * the Qwen3-8B layer at 1 and 32 rows). */

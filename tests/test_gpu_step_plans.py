@@ -10,7 +10,11 @@ from __future__ import annotations
 
 import ctypes
 import math
+import os
+import subprocess
+import sys
 import time
+from pathlib import Path
 
 import pytest
 import torch
@@ -317,3 +321,50 @@ def test_moe_replays_prepare_in_the_same_time_at_every_capacity(device):
         print(f"host us per replay: {small:.1f} at 64 rows, {large:.1f} at {capacity // 2 + 1}", flush=True)
         # The search over this capacity's row counts, twice a replay, took it from 45 to 96 us.
         assert large <= 1.5 * small
+
+
+# A program of its own, so that the HIP runtime logs its calls.
+GRAPH_PROGRAM = """
+import sys
+import torch
+from crosspool_amd.agent import FfnAgent
+from crosspool_amd.moe import MoeFfnWeights, MoeLayerSpec, MoeRouterWeights
+from crosspool_amd.weights import DenseFfnWeights
+
+device = torch.device("cuda:0")
+
+
+def normal(*shape):
+    return (torch.randn(shape, device=device) * 0.05).bfloat16()
+
+
+pool = normal(512, 256)
+slots = torch.arange(512, device=device, dtype=torch.int32)
+with FfnAgent(device, graph_dispatch=sys.argv[1] == "capture") as agent:
+    agent.register_layer(instance_index=0, layer_ordinal=0, weights=DenseFfnWeights.from_tensors(normal(512, 256), normal(256, 256)))
+    agent.register_moe_layer(instance_index=0, layer_ordinal=1, spec=MoeLayerSpec(routed_expert_count=8, routed_topk=2),
+                             weights=MoeFfnWeights(normal(8, 256, 256), normal(8, 256, 128), MoeRouterWeights(normal(8, 256))))
+    agent.materialize(maximum_row_capacity=512)
+    agent.lanes[0].set_graph_dispatch(True)
+    print("REPLAYS", file=sys.stderr, flush=True)
+    for rows in (1, 64, 65, 100, 128, 129, 193, 256, 257, 321, 400, 512):
+        for ordinal in (0, 1):
+            agent.execute(instance_index=0, layer_ordinal=ordinal, pool=pool, slots=slots, rows=rows)
+    agent.check_health()
+    print("END", file=sys.stderr, flush=True)
+"""
+
+
+@pytest.mark.parametrize("switched_on", ("capture", "later"))
+def test_graph_dispatch_instantiates_no_graph_in_a_replay(switched_on):
+    print(f"graph dispatch switched on at {switched_on}", flush=True)
+    root = Path(__file__).resolve().parent.parent
+    result = subprocess.run(
+        [sys.executable, "-c", GRAPH_PROGRAM, switched_on], cwd=root, capture_output=True, text=True, timeout=100,
+        env={**os.environ, "PYTHONPATH": str(root), "AMD_LOG_LEVEL": "3"},
+    )
+    assert result.returncode == 0, result.stderr[-2000:]
+    before, after = result.stderr.split("REPLAYS\n")
+    replays, rest = after.split("END\n")
+    assert before.count("hipGraphInstantiate") > 0 and replays.count("hipGraphLaunch") > 0
+    assert replays.count("hipGraphInstantiate") == 0 and replays.count("hipGraphCreate") == 0
