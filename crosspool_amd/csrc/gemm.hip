@@ -422,6 +422,34 @@ double step_us(const GemmChoice &choice, int64_t rows, int64_t n, int64_t k, dou
   return us;
 }
 
+// The model's time of one launch over `splits` K ranges, or -1 where they would be too short or
+// the last one empty.
+double step_split_us(const StepTile &tile, int64_t rows, int64_t n, int64_t k, int64_t splits) {
+  const int64_t slabs = (k + 63) / 64;
+  const int64_t per_range = (slabs + splits - 1) / splits;
+  if (splits > 1 && (per_range < kStepMinSlabs || (splits - 1) * per_range >= slabs)) {
+    return -1.0;
+  }
+  const double stream = 2.0 * static_cast<double>(n) * static_cast<double>(k) / kStepWeightBytesPerUs;
+  const double plane_us = 8.0 * static_cast<double>(rows * n) / kStepPartialBytesPerUs;
+  return kStepLaunchUs + stream + step_compute_us(tile, rows, n, per_range, splits) +
+         (splits > 1 ? kStepReduceUs + static_cast<double>(splits) * plane_us : 0.0);
+}
+
+// Whether choose_step_tile can take a K split: none of its unsplit launches is cheaper.
+bool step_split_pays(int64_t rows, int64_t n, int64_t k) {
+  double unsplit = -1.0;
+  double split = -1.0;
+  for (const StepTile &tile : kStepTiles) {
+    for (const int64_t splits : kStepSplits) {
+      const double us = step_split_us(tile, rows, n, k, splits);
+      double &least = splits > 1 ? split : unsplit;
+      least = us >= 0.0 && (least < 0.0 || us < least) ? us : least;
+    }
+  }
+  return split >= 0.0 && split <= unsplit;
+}
+
 GemmChoice choose_step_tile(const GemmChoice &base, int64_t rows, int64_t n, int64_t k) {
   const int64_t slabs = (k + 63) / 64;
   GemmChoice best = base;
@@ -431,17 +459,11 @@ GemmChoice choose_step_tile(const GemmChoice &base, int64_t rows, int64_t n, int
   }
   double best_us = base_us * (1.0 - kStepGain);
   const double stream = 2.0 * static_cast<double>(n) * static_cast<double>(k) / kStepWeightBytesPerUs;
-  const double plane_us = 8.0 * static_cast<double>(rows * n) / kStepPartialBytesPerUs;
   for (const StepTile &tile : kStepTiles) {
     for (const int64_t splits : kStepSplits) {
-      const int64_t per_range = (slabs + splits - 1) / splits;
-      if (splits > 1 && (per_range < kStepMinSlabs || (splits - 1) * per_range >= slabs)) {
-        continue;  // ranges too short, or the last one empty
-      }
-      const double us = kStepLaunchUs + stream + step_compute_us(tile, rows, n, per_range, splits) +
-                        (splits > 1 ? kStepReduceUs + static_cast<double>(splits) * plane_us : 0.0);
-      if (us < best_us) {
-        best = {GemmKind::Tile, tile.variant, splits > 1 ? per_range * 64 : k, splits};
+      const double us = step_split_us(tile, rows, n, k, splits);
+      if (us >= 0.0 && us < best_us) {
+        best = {GemmKind::Tile, tile.variant, splits > 1 ? (slabs + splits - 1) / splits * 64 : k, splits};
         best_us = us;
       }
     }
@@ -550,6 +572,17 @@ GemmChoice choose_dense_gate_up(int64_t capacity, int64_t n, int64_t k, bool &fu
 
 GemmChoice refine_dense_choice(const GemmChoice &base, int64_t rows, int64_t n, int64_t k) {
   return base.kind == GemmKind::Tile && rows >= kStepMinRows ? choose_step_tile(base, rows, n, k) : base;
+}
+
+size_t refined_scratch_bytes(int64_t capacity, int64_t n, int64_t k) {
+  // A column split keeps no sums, so where neither choice splits K without one, neither does
+  // with one; pricing those is most of a choice's host time at many rows.
+  const GemmChoice whole = choose_gemm(capacity, n, k, false, false);
+  if (whole.kind == GemmKind::Tile && whole.k_split == 1 &&
+      (capacity < kStepMinRows || !step_split_pays(capacity, n, k))) {
+    return 0;
+  }
+  return gemm_scratch_bytes(refine_dense_choice(choose_gemm(capacity, n, k, false), capacity, n, k), capacity, n, k);
 }
 
 // The tile and K split of a biased projection at `rows` rows (unsplit when `scratch_bytes` has no

@@ -18,6 +18,7 @@
 #include <cstring>
 #include <memory>
 #include <mutex>
+#include <optional>
 #include <string>
 #include <vector>
 
@@ -1516,7 +1517,7 @@ size_t xp_projection_workspace_bytes(int64_t rows, int64_t n, int64_t k, int dty
     return most;
   }
   for (int64_t capacity = 8; capacity <= tuned_projection_rows(rows); capacity += capacity < 64 ? capacity : 64) {
-    most = std::max(most, gemm_scratch_bytes(choose_tuned_projection(capacity, n, k), capacity, n, k));
+    most = std::max(most, refined_scratch_bytes(capacity, n, k));
     if (capacity >= kExtendedMinRows) {
       double us = 0.0;
       most = std::max(most, gemm_scratch_bytes(choose_extended(capacity, n, k, static_cast<size_t>(INT64_MAX), us),
@@ -1559,7 +1560,13 @@ int xp_projection_split(const void *x, int64_t rows, int64_t k, const void *w, i
   args.k = k;
   args.dtype = dtype;
   const size_t scratch_bytes = workspace != nullptr ? workspace_bytes : 0;
-  const ProjectionPlan plan = plan_projection(rows, n, k, static_cast<int>(element), scratch_bytes);
+  std::optional<ProjectionPlan> general;  // the general kernel's, where it is asked for
+  const auto plan = [&]() -> const ProjectionPlan & {
+    if (!general) {
+      general = plan_projection(rows, n, k, static_cast<int>(element), scratch_bytes);
+    }
+    return *general;
+  };
   if (tuned_projection_shape(n, k, dtype) && aligned16(x) && aligned16(w) && aligned16(out) &&
       (args.act.gated || args.act.function == kActivationNone)) {
     const bool gated = args.act.gated != 0;
@@ -1589,7 +1596,7 @@ int xp_projection_split(const void *x, int64_t rows, int64_t k, const void *w, i
     } else if (rows >= kExtendedMinRows) {
       double us = 0.0;
       const GemmChoice choice = choose_extended(capacity, n, k, scratch_bytes, us);
-      if (us < plan.us) {
+      if (us < plan().us) {
         XP_HIP_CHECK(launch(make_extended_gemm(gemm, capacity, gated, choice), hip_stream));
         if (choice.k_split > 1) {
           args.partials = gemm.partials;
@@ -1600,8 +1607,8 @@ int xp_projection_split(const void *x, int64_t rows, int64_t k, const void *w, i
       }
     }
   }
-  args.partials = plan.ranges > 1 ? static_cast<float *>(workspace) : nullptr;
-  const ProjectionLaunch kernels = make_projection(args, plan, rows, dtype);
+  args.partials = plan().ranges > 1 ? static_cast<float *>(workspace) : nullptr;
+  const ProjectionLaunch kernels = make_projection(args, plan(), rows, dtype);
   XP_HIP_CHECK(launch(kernels.main, static_cast<hipStream_t>(stream)));
   XP_HIP_CHECK(launch(kernels.reduce, static_cast<hipStream_t>(stream)));
   return XP_OK;

@@ -425,6 +425,8 @@ GemmChoice choose_dense_gate_up(int64_t capacity, int64_t n, int64_t k, bool &fu
 GemmChoice refine_dense_choice(const GemmChoice &base, int64_t rows, int64_t n, int64_t k);
 // The choice for a projection that has no scratch: it leaves no partial sums of K ranges.
 GemmChoice choose_unsplit(int64_t rows, int64_t n, int64_t k);
+// Scratch of choose_gemm's choice for an ungated projection, refined at the same rows.
+size_t refined_scratch_bytes(int64_t capacity, int64_t n, int64_t k);
 // Whether choose_gemm's kernel for an ungated projection at `capacity` rows can take the
 // mailbox gather fused: the split kernel with one token group and K <= 4096 (the MoE step's
 // router projection then gathers and normalises the rows itself).
