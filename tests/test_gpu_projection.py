@@ -190,6 +190,93 @@ def test_aligned_projections(device, dtype, epilogue):
                 _assert_within_bound(out, x, w, bias)
 
 
+# The other epilogues of the same routes: ReLU, GELU by erf and its tanh approximation, and Gates
+# without a limit, where the tile kernels or the general one apply them and over K ranges.
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))
+@pytest.mark.parametrize("biased", (False, True))
+@pytest.mark.parametrize("function", ("silu", "relu", "gelu", "gelu_tanh"))
+@pytest.mark.parametrize("limit", (None, 1.5))
+def test_aligned_projection_activations(device, dtype, biased, function, limit):
+    code = {"silu": _native.XP_ACTIVATION_SILU, "relu": _native.XP_ACTIVATION_RELU}.get(function, _native.XP_ACTIVATION_GELU)
+    desc = _native.ActivationDesc()
+    desc.function, desc.approximate_tanh, desc.alpha, desc.gated = code, int(function == "gelu_tanh"), 1.25, 1
+    desc.has_limit, desc.limit, desc.up_offset = int(limit is not None), limit or 0.0, 0.25
+    for rows, k, n in ((64, 2048, 2064), (65, 2048, 8208), (130, 2048, 2064), (257, 4096, 4112), (700, 1000, 8192)):
+        print(f"activation {dtype} biased={biased} {function} limit={limit} {rows}x{n}x{k}", flush=True)
+        x, w, bias, _ = _operands(device, rows, k, n, dtype)
+        w.mul_(k**-0.5)
+        projected = x.double() @ w.double().t() + (bias.double() if biased else 0.0)
+        gate, up = projected.to(dtype).double()[:, 0::2], projected.to(dtype).double()[:, 1::2]
+        if limit is not None:
+            gate, up = gate.clamp(max=limit), up.clamp(-limit, limit)
+        if function == "silu":
+            act = gate / (1.0 + torch.exp(-1.25 * gate))
+        elif function == "relu":
+            act = gate.clamp(min=0.0)
+        else:
+            act = torch.nn.functional.gelu(gate, approximate="tanh" if function == "gelu_tanh" else "none")
+        expected = act * (up + 0.25)
+        nbytes = _native.library().xp_projection_workspace_bytes(rows, n, k, CODES[dtype])
+        workspace = torch.empty(max(nbytes, 16), device=device, dtype=torch.uint8)
+        for size in sorted({0, nbytes}):
+            out = torch.full((rows, n // 2), 7.0, device=device, dtype=dtype)
+            _native.call(
+                "xp_projection_split", _pointer(x), rows, k, _pointer(w), n, _pointer(bias) if biased else None, _pointer(out),
+                CODES[dtype], ctypes.byref(desc), _pointer(workspace) if size else None, size,
+                ctypes.c_void_p(torch.cuda.current_stream().cuda_stream),
+            )
+            torch.cuda.synchronize()
+            # One rounding of the output and the few activations whose input rounds the other way.
+            error = (out.double() - expected).norm() / expected.norm()
+            assert error <= 2.0 ** -(MANTISSA[dtype] + 1), f"{rows}x{n}x{k} workspace {size}: {error:.2e}"
+
+
+# Infinities and NaN stay in their rows and columns on every route: K ends inside a slab and rows
+# and weight rows inside tiles, where a kernel's padding must not meet them.
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float16))
+@pytest.mark.parametrize("epilogue", ("none", "bias", "silu", "bias+silu", "relu", "bias+gelu"))
+def test_aligned_projections_keep_infinities_and_nan_in_their_rows(device, dtype, epilogue):
+    gated = epilogue not in ("none", "bias")
+    desc = _native.ActivationDesc()
+    desc.function = (_native.XP_ACTIVATION_GELU if "gelu" in epilogue else _native.XP_ACTIVATION_RELU if "relu" in epilogue
+                     else _native.XP_ACTIVATION_SILU)
+    desc.alpha, desc.gated = 1.0, 1
+    for rows, k, n in ((7, 1000, 528), (13, 2056, 272), (40, 1000, 528), (70, 1000, 528), (130, 2056, 2064), (300, 3000, 1040)):
+        print(f"infinities {dtype} {epilogue} {rows}x{n}x{k}", flush=True)
+        x, w, bias, _ = _operands(device, rows, k, n, dtype)
+        w.mul_(k**-0.5)
+        # the first and last columns of rows inside and at the end of a tile
+        x[2, 0], x[4, k - 1], x[rows - 1, 5], w[n - 1, 3], w[33, k - 1] = (
+            float("inf"), float("nan"), float("-inf"), float("inf"), float("nan"))
+        bias = bias if "bias" in epilogue else None
+        projected = x.float().cpu() @ w.float().cpu().t() + (0.0 if bias is None else bias.cpu())
+        expected = projected
+        if gated:
+            gate, up = projected.to(dtype).float()[:, 0::2], projected.to(dtype).float()[:, 1::2]
+            if "relu" in epilogue:
+                act = torch.where(gate.isnan() | (gate > 0), gate, torch.zeros_like(gate))
+            elif "gelu" in epilogue:
+                act = 0.5 * gate * (1.0 + torch.erf(gate * 0.5**0.5))
+            else:
+                act = gate / (1.0 + torch.exp(-gate))
+            expected = act * up
+        expected = expected.to(dtype).float()
+        nbytes = _native.library().xp_projection_workspace_bytes(rows, n, k, CODES[dtype])
+        workspace = torch.empty(max(nbytes, 16), device=device, dtype=torch.uint8)
+        for size in sorted({0, nbytes}):
+            out = torch.full((rows, n // 2 if gated else n), 7.0, device=device, dtype=dtype)
+            _native.call(
+                "xp_projection_split", _pointer(x), rows, k, _pointer(w), n, _pointer(bias), _pointer(out), CODES[dtype],
+                ctypes.byref(desc) if gated else None, _pointer(workspace) if size else None, size,
+                ctypes.c_void_p(torch.cuda.current_stream().cuda_stream),
+            )
+            torch.cuda.synchronize()
+            got = out.float().cpu()
+            assert torch.equal(torch.isnan(got), torch.isnan(expected)), f"{rows}x{n}x{k} workspace {size}"
+            assert torch.equal(torch.isinf(got), torch.isinf(expected))
+            assert torch.equal(got[torch.isinf(got)], expected[torch.isinf(expected)])
+
+
 # A SiLU epilogue is evaluated with expf and an IEEE divide whichever kernel the row count, the
 # bias and the workspace choose.  Every row of x is a unit vector, so the projected values are the
 # weights themselves and only the activation and the store round (alpha is a power of two).  The

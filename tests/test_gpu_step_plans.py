@@ -21,7 +21,7 @@ import torch
 
 from crosspool_amd import _native
 from crosspool_amd.agent import ExecutorLane, FfnAgent
-from crosspool_amd.ffn import RouterProjectionPrecision
+from crosspool_amd.ffn import GeluActivation, ReluActivation, RouterAlgorithm, RouterProjectionPrecision, SiluActivation
 from crosspool_amd.moe import MoeFfnWeights, MoeLayerSpec, MoeRouterWeights
 from crosspool_amd.weights import DenseFfnWeights
 
@@ -243,6 +243,61 @@ def test_moe_steps_between_capacities(device, capacity, rows_list):
         # Two route roundings, the combine's and flipped activations; a logit at a rounding
         # boundary may pick another expert in a few rows.
         assert difference.median() <= 2.0**-7 and (difference > 2.0**-5).float().mean() <= 0.01, f"{rows} rows"
+
+
+# The same with what a MoE layer can add to the plain one: a sigmoid Router with a correction, a
+# shared expert, projection biases, another activation and a scaling factor.
+@pytest.mark.parametrize("activation", (SiluActivation(), ReluActivation(), GeluActivation("none")))
+def test_moe_steps_of_extended_layers(device, activation):
+    hidden, intermediate, routed, topk, capacity, scaling = 256, 128, 8, 2, 1024, 2.5
+    experts = routed + 1
+    generator = torch.Generator(device=device).manual_seed(3)
+
+    def normal(*shape, std=1.0):
+        return torch.randn(shape, device=device, generator=generator) * std
+
+    correction = normal(routed, std=0.1)
+    weights = MoeFfnWeights(
+        normal(experts, 2 * intermediate, hidden, std=0.05).bfloat16(), normal(experts, hidden, intermediate, std=0.05).bfloat16(),
+        MoeRouterWeights(normal(routed, hidden, std=0.05), correction),
+        normal(experts, 2 * intermediate, std=0.2), normal(experts, hidden, std=0.2))
+    pool = normal(capacity + 8, hidden).bfloat16()
+    slots = torch.randperm(pool.shape[0], device=device).to(torch.int32)
+    x = pool.double()
+    scores = torch.sigmoid(x @ weights.router.projection.double().t())
+    ids = (scores + correction.double()).topk(topk, dim=1).indices
+    picked = scores.gather(1, ids)
+    share = torch.zeros((x.shape[0], experts), dtype=torch.float64, device=device)
+    share.scatter_(1, ids, picked / picked.sum(1, keepdim=True))
+    share[:, routed] = 1.0 / scaling
+    expected = torch.zeros_like(x)
+    for expert in range(experts):
+        projected = x @ weights.i_proj[expert].double().t() + weights.i_proj_bias[expert].double()
+        gate, up = projected.bfloat16().double()[:, 0::2], projected.bfloat16().double()[:, 1::2]
+        function = {SiluActivation: torch.nn.functional.silu, ReluActivation: torch.relu,
+                    GeluActivation: torch.nn.functional.gelu}[type(activation)]
+        y = (function(gate) * up).bfloat16().double() @ weights.o_proj[expert].double().t() + weights.o_proj_bias[expert].double()
+        expected += scaling * y * share[:, expert: expert + 1]
+    spec = MoeLayerSpec(routed_expert_count=routed, routed_topk=topk, shared_expert_count=1, routed_scaling_factor=scaling,
+                        router_algorithm=RouterAlgorithm.SIGMOID, activation=activation,
+                        router_projection_precision=RouterProjectionPrecision.FP32)
+    with FfnAgent(device) as agent:
+        agent.register_moe_layer(instance_index=0, layer_ordinal=0, weights=weights, spec=spec)
+        agent.materialize(maximum_row_capacity=capacity)
+        # 16-route, 64-, 128- and 256-row expert tiles, plans below and at a capacity
+        for rows in (1, 8, 9, 64, 65, 140, 256, 300, 577, 1000, 1024):
+            print(f"extended moe step {type(activation).__name__} {rows}/{capacity}", flush=True)
+            out = torch.zeros_like(pool)
+            agent.execute(instance_index=0, layer_ordinal=0, pool=pool, slots=slots, rows=rows, out_pool=out)
+            agent.check_health()
+            live = slots[:rows].long()
+            difference = (out[live].double() - expected[live]).norm(dim=1) / expected[live].norm(dim=1)
+            # Two route roundings, the combine's and flipped activations; a score within 2^-20 of
+            # another may pick another expert in a few rows.
+            assert difference.median() <= 2.0**-7 and (difference > 2.0**-5).double().mean() <= 0.01, f"{rows} rows"
+            untouched = torch.ones(pool.shape[0], dtype=torch.bool, device=device)
+            untouched[live] = False
+            assert not out[untouched].any()
 
 
 @pytest.mark.parametrize("precision", (RouterProjectionPrecision.FP32, RouterProjectionPrecision.FP32_LOGITS))
