@@ -1622,13 +1622,20 @@ __device__ __forceinline__ void static_for(F &&f) {
 // token and weight tiles in its L2, and every weight tile is fetched by one XCD in one
 // round (Qwen3-8B gate_up at 2048 rows: 612 instead of 968 MB fetched per launch, same
 // time).  Weight tiles that do not split evenly are given out in runs of consecutive tiles of
-// such blocks instead (in grid order every token tile's copy of a weight tile was on another
-// XCD): gate_up of the Qwen3-32B TP shard (25 tiles of 256) at 2048 / 8192 rows 126 -> 119 and
-// 470 -> 461 us, of a hidden-1536 layer (70) at 896 rows on 128 x 256 tiles 67.6 -> 55.8,
-// Qwen3-4B down (10) at 4096 rows 207 -> 194; worst Qwen3-4B gate_up (76) at 2048 rows, 184 ->
-// 188.  With more than 8 token tiles and even weight tiles the grid coordinates are used as
-// they are (blocks took 3 % longer; runs 2 % less on 256 x 256 tiles, 5 % more on 256 x 128), and
-// so are those of a single row or column of tiles, where there is nothing to share.
+// such blocks instead (in grid order the token tiles' copies of a weight tile are on 2, 4 or 8
+// XCDs).  A block is no larger than the run: of a grid of less than a round a run inside a larger
+// block is one token tile's, with a weight tile of its own for every workgroup.  Microseconds in
+// grid order / in runs: gate_up of the Qwen3-32B TP shard (25 weight tiles of 256) at 2048 rows
+// 129 / 119, of a hidden-1536 layer (140 of 128) at 163 rows 32.0 / 25.7, at 787 rows 74 / 64;
+// down of a hidden-896 layer (7 of 128) at 1024 rows 31.3 / 23.2; in runs of blocks as wide as
+// they go / of blocks that fit, with K splits: Qwen3-4B down (20) at 163 rows 27.1 / 31.8 / 26.0, at
+// 275 rows 32.4 / 36.0 / 31.0, hidden-1536 down (12) at 512 rows 31.2 / 32.5 / 27.4.  Runs of fewer
+// than four tiles stay on the widest blocks (hidden-1536 down, 12 x 2, at 256 rows 26.0 / 23.3 /
+// 25.6).  Slower than in grid order, of 1284 layers and projections at 17 to 4096 rows: down 3072 x
+// 8192 (12 x 2) at 512 rows 37.5 / 39.0, a hidden-896 layer at 65 to 128 rows by 2 %.  With more
+// than 8 token tiles and even weight tiles the grid coordinates are used as they are (blocks took
+// 3 % longer; runs 2 % less on 256 x 256 tiles, 5 % more on 256 x 128), and so are those of a single
+// row or column of tiles, where there is nothing to share.
 // The results are wave-uniform; readfirstlane keeps them (and the buffer resources built from
 // them) in scalar registers.
 __device__ __forceinline__ void tile_coordinates(int &tn, int &tm) {
@@ -1659,7 +1666,14 @@ __device__ __forceinline__ void tile_coordinates(int &tn, int &tm) {
   const int band = place / (8 * nx);
   const int in_band = place - band * 8 * nx;
   const int rows = ny - 8 * band < 8 ? ny - 8 * band : 8;
-  const int block_tiles = 32 / rows;
+  // The fewest weight tiles (at most 32 / rows) whose block holds the run and is at least as
+  // wide as high; short runs keep the widest.
+  const int run = (total + 7) / 8;
+  int block_tiles = 32 / rows;
+  while (run >= 4 && block_tiles > 1 && (block_tiles - 1) * (block_tiles - 1) >= run &&
+         (block_tiles - 1) * rows >= run) {
+    --block_tiles;
+  }
   const int block = in_band / (block_tiles * rows);
   const int rest = in_band - block * block_tiles * rows;
   const int tiles = nx - block * block_tiles < block_tiles ? nx - block * block_tiles : block_tiles;

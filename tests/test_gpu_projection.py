@@ -315,3 +315,23 @@ def test_silu_epilogues_are_evaluated_in_full_precision(device, dtype, alpha, ga
         share = (out.cpu() != expected).double().mean().item()
         bound = 2 * 2.5 * 2.0**-24 / 2.0 ** -(MANTISSA[dtype] + 1)
         assert share <= bound, f"workspace {size}: share of other roundings {share:.2e} of at most {bound:.2e}"
+
+
+# Grids whose weight tiles do not split over the XCDs: every tile is computed once, whatever the
+# blocks of an XCD's run (runs shorter than a block, one band of 8 token tiles and several).
+@pytest.mark.parametrize("n", (384, 640, 896, 1536, 2568, 3328))
+def test_tile_order_covers_every_tile(device, n):
+    k = 520
+    generator = torch.Generator(device=device).manual_seed(n)
+    w = (torch.randn((n, k), device=device, generator=generator) * k**-0.5).bfloat16()
+    for rows in (65, 130, 163, 275, 358, 520, 700, 1100, 2100):
+        print(f"tile order {rows}x{n}x{k} {_native.gemm_variant(rows, n, k, False)}", flush=True)
+        x = torch.randn((rows, k), device=device, generator=generator).bfloat16()
+        out = torch.full((rows, n), 7.0, device=device, dtype=torch.bfloat16)
+        nbytes = _native.gemm_workspace_bytes(rows, n, k, False)
+        workspace = torch.empty(max(nbytes, 16), device=device, dtype=torch.uint8)
+        _native.call("xp_gemm_down", _pointer(x), rows, k, _pointer(w), n, _pointer(out), None, rows,
+                     _pointer(workspace) if nbytes else None, nbytes,
+                     ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        _assert_within_bound(out, x, w, None)
