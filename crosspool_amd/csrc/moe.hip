@@ -505,32 +505,41 @@ int moe_tile_rows(MoeTile tile) { return tile == MoeTile::Small ? grouped_split_
 // 16-route tiles; more take the grouped tile kernel on the shortest expert tile that holds most
 // experts' routes.  An expert's weights are read once per tile of its routes, and the LDS a
 // tile's token rows do not take holds weight slabs in flight (the grouped projections are bound
-// by the weight bytes each CU has in flight).  The thresholds are about where neighbours cross,
-// by routes per expert on average (layer us at the Qwen3-30B-A3B shape, 128 experts, top-8, then
-// of a 1024 x 512, 64-expert top-6 layer): 16-route tiles against 64-row ones (two workgroups per
-// CU) at 3 / 4 / 8 routes 207 / 218 / 256 and 233 / 238 / 245, at 3.8 / 6 routes 63.0 / 65.8
-// and 60.0 / 61.3; those against 128-row ones with nontemporal weight loads at 40 / 48 / 56
-// routes 268 / 289 / 318 and 300 / 307 / 312, at 36 / 60 routes 65.9 / 88.8 and 69.6 / 73.7;
-// those against 128-row ones with plain loads (an expert split over two tiles finds its weights
-// in the last-level cache for the second) at 96 / 112 / 128 routes 355 / 380 / 457 and 366 / 379
-// / 396; and those against 256-row ones at 128 / 144 / 160 routes 396 / 443 / 485 and 424 / 431
-// / 463.  Experts of less than kRereadExpertBytes of gate_up weights gain nothing from the
-// second reading: 108 / 120 / 144 routes 114.1 / 111.6 / 118.7 on 128-row tiles against 102.0 /
-// 107.5 / 114.4 on 256-row ones.  192-row tiles were the fastest only there (106.9 / 112.2 at
-// 120 / 144; the large layer at 128 routes 431).
+// by the weight bytes each CU has in flight).  Every tile was forced at 3 to 160 routes per expert
+// on eight layers (hidden x intermediate, experts, top-k).  Neighbours cross at, in routes per
+// expert on average:
+//                             16 -> 64   64 -> 128 nt   -> 128   -> 256
+//   2048 x 768, 128, 8           > 5           55          107     135
+//   2048 x 1024, 64, 8           > 5           57          111     130
+//   4096 x 1536, 32, 4             4           48            -      99
+//   1536 x 768, 64, 8            > 5           57            -     119
+//   2048 x 512, 64, 8            > 5           49            -     110
+//   1024 x 768, 64, 8              5           51          115     118
+//   1024 x 512, 64, 6              3           45            -     103
+//   1024 x 256, 64, 8              4           49           50     130
+// (128 nt: 128-row tiles with nontemporal weight loads; with plain loads an expert split over two
+// tiles finds its weights in the last-level cache for the second.)  Where they cross follows the
+// rounds of workgroups as much as the expert's size, which the rule does not price: experts of at
+// most kRereadExpertBytes of gate_up weights take 128-row tiles from 46 routes instead of 52 (1024
+// x 512 at 48: 78.3 us on 64-row, 73.5 on 128-row tiles) and 256-row tiles right after the
+// nontemporal ones, since a second reading costs them nothing (at 144: 112.8 and 106.7); larger ones
+// keep 128-row tiles up to 136 (2048 x 768 at 128: 390 us, on 256-row tiles 412).  Over these layers
+// the rule's choice costs 0.9 % more than the best tile on average; most, 16 %, where 4096 x 1536 at
+// 136 routes takes 402 us on 128-row tiles and would 347 on 256-row ones.
 constexpr int64_t kRereadExpertBytes = int64_t{4} << 20;
 
 MoeTile choose_moe_tile(int64_t routes, int64_t experts, int64_t gate_up_bytes) {
+  const bool small = gate_up_bytes <= kRereadExpertBytes;
   if (routes <= 4 * experts) {
     return MoeTile::Small;
   }
-  if (routes <= 52 * experts) {
+  if (routes <= (small ? 46 : 52) * experts) {
     return MoeTile::Rows64;
   }
   if (routes <= 104 * experts) {
     return MoeTile::Rows128Stream;
   }
-  return routes <= 136 * experts && gate_up_bytes >= kRereadExpertBytes ? MoeTile::Rows128 : MoeTile::Rows256;
+  return routes <= 136 * experts && !small ? MoeTile::Rows128 : MoeTile::Rows256;
 }
 
 template <class P>
