@@ -351,7 +351,7 @@ GemmChoice choose_gemm(int64_t capacity, int64_t n, int64_t k, bool gated, bool 
 // clocks higher and its L2s have fewer readers); the weights' stream adds to it, since a round's
 // tiles wait for the same lines; a K split adds its reduction and its sums' traffic.  A
 // column split is two such launches.
-// Fitted (log least squares) to 9400 forced choices on MI355X: Qwen3 0.6B / 1.7B / 4B / 8B, a
+// Fitted (log least squares) to some 9500 forced choices on MI355X: Qwen3 0.6B / 1.7B / 4B / 8B, a
 // hidden-1536 layer and the Qwen3-32B TP shard, both projections, 26 row counts from 65 to 4096,
 // every shape and 1 to 16 K ranges, weights streamed from HBM: mean error 6.1 %, and its picks
 // sum to 0.6 % above the fastest measured single launch of each.  The column splits it prices

@@ -262,8 +262,8 @@ constexpr int kSplitMaxGroups = 2;
 //
 // HALVES: 8-row halves of a weight block per wave.  One instead of two doubles the workgroups of
 // a projection whose 16-row blocks leave half the CUs idle; the K ranges and their order are the
-// same, and so are the bits.  Captured 28-layer Qwen3-0.6B stack at 7 rows (96 and 64 workgroups
-// before) 518 -> 469 us; Qwen3-1.7B layer at 1 / 4 rows (down: 128) 24.4 / 25.2 -> 21.6 / 22.2.
+// same, and so are the bits.  Captured 28-layer Qwen3-0.6B stack at 7 rows (down on 128 workgroups
+// instead of 64; gate_up keeps its 192) 518 -> 469 us; Qwen3-1.7B layer at 1 / 4 rows (down: 128) 24.4 / 25.2 -> 21.6 / 22.2.
 template <int DEPTH, int TG, bool GATED, bool GATHER = false, class P = Bf16Payload, int HALVES = 2>
 __global__ __launch_bounds__(64 * kSplitWaves) void split_gemm_kernel(GemmArgs a) {
   constexpr int ROWS = 8 * HALVES;  // weight rows of a block

@@ -1,5 +1,5 @@
 // General projections and the standalone activation: the FfnAgent operator cases that the
-// bf16 MFMA kernels of gemm.hip do not take.
+// tuned kernels of gemm.hip do not take.
 //
 // Reference behaviour (CrossPool checkout):
 //  * Gemm.run_into (src/xpool/runtime/ffnagent/operators/linear.py:163-257) with the
@@ -15,9 +15,11 @@
 //    every other non-positive value to +0 (activation.py:19-27).
 //
 // Payloads are bf16, fp16 or fp32 (activations: bf16 or fp16), any K and N, rows of any
-// alignment: the shapes, dtypes, biases and epilogues of the reference's operator contract
-// beside the Qwen3 hot path (bf16, no bias, SiLU, aligned), which gemm.hip serves.  The
-// Router's FP32 and FP32_LOGITS projections run here too.
+// alignment.  16-bit projections of whole 16-byte rows leave this file where gemm.hip serves them:
+// without a bias or activation the Dense projection kernels, from 65 rows with a bias or a gated
+// activation the tile kernels' EXTENDED epilogue when it is modelled as faster (and
+// projection_reduce_kernel for its K ranges); a gated activation evaluates as here on every route.
+// The Router's FP32 and FP32_LOGITS projections, and its odd geometries, run here too.
 
 #include "xp_kernels.hpp"
 
@@ -558,7 +560,6 @@ ProjectionLaunch make_projection(const ProjectionArgs &args, const ProjectionPla
   ProjectionLaunch launches;
   ProjectionArgs record = args;
   record.k_slice = plan.k_slice;
-  launches.ranges = plan.ranges;
   launches.main.func = args.dtype == kDtypeF32
                            ? (x_dtype == kDtypeF32   ? projection_kernel_for<F32Payload, F32Payload>(plan.tile)
                               : x_dtype == kDtypeF16 ? projection_kernel_for<F16Payload, F32Payload>(plan.tile)

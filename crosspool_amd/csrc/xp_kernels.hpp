@@ -319,7 +319,6 @@ size_t projection_scratch_bytes(int64_t capacity, int64_t n, int64_t k, int elem
 struct ProjectionLaunch {
   KernelLaunch main;
   KernelLaunch reduce;
-  int64_t ranges = 1;
 };
 // Grids for `capacity` rows.  x_dtype: the tokens' dtype, args.dtype except for 16-bit tokens
 // against fp32 weights.

@@ -13,9 +13,9 @@ Mirrors the reference's operator layer (CrossPool checkout):
 Every launch goes to the HIP library on the current torch stream and allocates nothing
 (the plan's workspace holds all scratch), so a ``run_into`` can be captured into a graph.
 Projections of bf16 payloads with aligned shapes, no bias and either no epilogue or the
-gated SiLU epilogue over INTERLEAVED rows take the MFMA kernels (``xp_gemm_down`` /
-``xp_gemm_gate_up_silu``); every other projection -- fp16 and fp32 payloads, odd K or N, a
-bias, ReLU / GELU epilogues -- takes ``xp_projection``.
+gated SiLU epilogue over INTERLEAVED rows take ``xp_gemm_down`` / ``xp_gemm_gate_up_silu``;
+every other projection -- fp16 and fp32 payloads, odd K or N, a bias, ReLU / GELU epilogues --
+takes ``xp_projection_split``.
 """
 
 from __future__ import annotations
@@ -154,7 +154,7 @@ class GemmPlan:
     output_layout: TensorLayout
     fused_activation: Activation | None
     workspace: WorkspaceLayout
-    kernel: str  # "gate_up_silu" or "down" (MFMA kernels) or "projection" (xp_projection)
+    kernel: str  # "gate_up_silu" or "down" (xp_gemm_*) or "projection" (xp_projection_split)
 
     @classmethod
     def prepare(
@@ -184,8 +184,9 @@ class GemmPlan:
         output_width = width // 2 if gated_epilogue else width
         if result_layout.shape != (rows, output_width):
             raise ValueError(f"GEMM result must be {(rows, output_width)}")
-        # The MFMA kernels take bf16 rows of 16-byte multiples, no bias, and at most 16384 columns
-        # on the side the C ABI treats as the hidden size (N for down, K for gate_up).
+        # xp_gemm_down and xp_gemm_gate_up_silu take bf16 rows of 16-byte multiples, no bias, and at
+        # most 16384 columns on the side the C ABI treats as the hidden size (N for down, K for
+        # gate_up).  xp_projection chooses among its own kernels and the tuned 16-bit ones.
         aligned = dtype is torch.bfloat16 and weight_layout.bias is None and hidden % 8 == 0 and width % 16 == 0
         if aligned and fused is None and width <= 16384:
             kernel = "down"

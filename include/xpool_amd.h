@@ -148,8 +148,9 @@ int xp_gemm_down(const void *activated, int64_t rows, int64_t intermediate, cons
  * (XP_DTYPE_BF16 / F16 / F32), bias fp32 [n] or NULL, any K and N, element-aligned rows.
  * The fp32 sum plus bias is stored rounded to the dtype; with an activation (NULL: none) it is
  * first rounded to the dtype (the projection rounding point), then activated in fp32, then
- * stored.  For the operator contract's shapes, dtypes and biases; bf16 SiLU projections of
- * aligned shapes without bias take xp_gemm_gate_up_silu / xp_gemm_down.  Replaces Gemm.run_into
+ * stored (SiLU with expf and an IEEE divide, whichever kernel serves the call; bf16 projections
+ * of aligned shapes without bias can take xp_gemm_gate_up_silu / xp_gemm_down instead, whose SiLU
+ * is the Dense templates').  Replaces Gemm.run_into
  * for unquantized weights (src/xpool/runtime/ffnagent/operators/linear.py:163-257,
  * operators/simt.py:13-80) with the epilogue of operators/activation.py:112-173. */
 int xp_projection(const void *x, int64_t rows, int64_t k, const void *w, int64_t n, const float *bias, void *out,
@@ -214,9 +215,9 @@ int xp_dense_step(const void *pool_in, void *pool_out, int64_t pool_rows, const 
 /* xp_dense_step without a workspace argument: the step's workspace (gathered batch,
  * activated intermediate, K-range partial sums) is a static 64 MiB device array of the
  * library, one per device, held until the process ends.  It allocates nothing: no
- * hipMalloc / hipFree, no allocating library call.  Steps needing more than 64 MiB
- * (xp_dense_workspace_bytes(rows, hidden, intermediate) > 64 MiB, e.g. Qwen3-8B past about
- * 512 rows) fail with XP_ERROR_CAPACITY.  Every call on one device shares the array and
+ * hipMalloc / hipFree, no allocating library call.  Steps whose kernel choices need more than
+ * 64 MiB at their row count (Qwen3-8B at 683 to 2037 rows, where K is split, and past 2048) fail
+ * with XP_ERROR_CAPACITY.  Every call on one device shares the array and
  * leaves its contents behind (no region needs to start cleared): calls that overlap in time
  * on one device race, so order them on one stream.  No counterpart in the reference; it is
  * for callers that cannot allocate device memory (code under stream capture, tight serving
