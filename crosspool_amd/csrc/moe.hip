@@ -518,25 +518,31 @@ int moe_tile_rows(MoeTile tile) { return tile == MoeTile::Small ? grouped_split_
 //   1024 x 512, 64, 6              3           45            -     103
 //   1024 x 256, 64, 8              4           49           50     130
 // (128 nt: 128-row tiles with nontemporal weight loads; with plain loads an expert split over two
-// tiles finds its weights in the last-level cache for the second.)  Where they cross follows the
-// rounds of workgroups as much as the expert's size, which the rule does not price: experts of at
-// most kRereadExpertBytes of gate_up weights take 128-row tiles from 46 routes instead of 52 (1024
-// x 512 at 48: 78.3 us on 64-row, 73.5 on 128-row tiles) and 256-row tiles right after the
-// nontemporal ones, since a second reading costs them nothing (at 144: 112.8 and 106.7); larger ones
-// keep 128-row tiles up to 136 (2048 x 768 at 128: 390 us, on 256-row tiles 412).  Over these layers
-// the rule's choice costs 0.9 % more than the best tile on average; most, 16 %, where 4096 x 1536 at
-// 136 routes takes 402 us on 128-row tiles and would 347 on 256-row ones.
+// tiles finds its weights in the last-level cache for the second.)  Experts of at most
+// kRereadExpertBytes of gate_up weights take 128-row tiles from 46 routes instead of 52 (1024 x 512
+// at 48: 78.3 us on 64-row, 73.5 on 128-row tiles) and 256-row tiles right after the nontemporal
+// ones, since a second reading costs them nothing (at 144: 112.8 and 106.7); larger ones keep
+// 128-row tiles up to 136 (2048 x 768 at 128: 390 us, on 256-row tiles 412).  Where small experts go
+// to 256 rows follows the rounds of workgroups: 128-row gate_up tiles of every expert that fill
+// whole rounds start another one with the first expert of more than 128 routes (1024 x 512 at 92 /
+// 104 routes 79.6 / 107.0 us, on 256-row tiles 102.8), others have room for some in their last
+// round (1024 x 768, one and a half rounds, at 112: 123.5 and 127.8, at 120: 143.4 and 129.2).  Larger
+// experts' rounds are not priced.  Over these layers the rule's choice costs 0.8 % more than the
+// best tile on average; most, 16 %, where 4096 x 1536 at 136 routes takes 402 us on 128-row tiles and
+// would 347 on 256-row ones.
 constexpr int64_t kRereadExpertBytes = int64_t{4} << 20;
+constexpr int64_t kMoeComputeUnits = 256;
 
-MoeTile choose_moe_tile(int64_t routes, int64_t experts, int64_t gate_up_bytes) {
-  const bool small = gate_up_bytes <= kRereadExpertBytes;
+MoeTile choose_moe_tile(int64_t routes, int64_t experts, int64_t hidden, int64_t intermediate) {
+  const bool small = 4 * hidden * intermediate <= kRereadExpertBytes;
+  const bool whole_rounds = experts * ((2 * intermediate + 255) / 256) % kMoeComputeUnits == 0;
   if (routes <= 4 * experts) {
     return MoeTile::Small;
   }
   if (routes <= (small ? 46 : 52) * experts) {
     return MoeTile::Rows64;
   }
-  if (routes <= 104 * experts) {
+  if (routes <= (small && !whole_rounds ? 116 : 104) * experts) {
     return MoeTile::Rows128Stream;
   }
   return routes <= 136 * experts && !small ? MoeTile::Rows128 : MoeTile::Rows256;

@@ -746,7 +746,7 @@ int make_experts_launches(const ExpertsBinding &b, int64_t capacity, int64_t pla
   uint16_t *route_out = reinterpret_cast<uint16_t *>(b.workspace + layout.route_out);
   const int64_t routes = b.rows * b.topk;
   const int64_t plan_routes = plan_rows * b.topk;
-  const MoeTile tile = choose_moe_tile(plan_routes, b.experts, 4 * b.intermediate * b.hidden);
+  const MoeTile tile = choose_moe_tile(plan_routes, b.experts, b.hidden, b.intermediate);
   const int tile_rows = moe_tile_rows(tile);
   const int max_tiles = moe_tile_bound(plan_routes, b.experts, tile_rows);
   XP_REQUIRE(max_tiles <= 65535, "too many expert tiles for one call");

@@ -252,8 +252,7 @@ struct MoeCombineArgs {
 // 256-row expert tiles (Rows128Stream: 128 rows with the weights loaded nontemporally).
 enum class MoeTile : int { Small = 0, Rows64 = 1, Rows128Stream = 2, Rows128 = 3, Rows256 = 4 };
 int moe_tile_rows(MoeTile tile);
-// gate_up_bytes: one expert's gate_up weights.
-MoeTile choose_moe_tile(int64_t routes, int64_t experts, int64_t gate_up_bytes);
+MoeTile choose_moe_tile(int64_t routes, int64_t experts, int64_t hidden, int64_t intermediate);
 
 KernelLaunch make_router_topk(const RouterTopkArgs &args);
 KernelLaunch make_finalize_routing(const FinalizeRoutingArgs &args);
